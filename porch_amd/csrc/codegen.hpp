@@ -184,6 +184,9 @@ namespace porch::cg {
     };
 
     kernel_code emit_gemm(const gemm_request& request);
+    // fp32 products on the bf16 matrix cores, each value split into three
+    // bf16 values (emit_gemm_split.cpp).
+    kernel_code emit_gemm_split(const gemm_request& request);
     // How many chunks of K the MFMA kernel should split a product into (1:
     // none): when its tiles cannot fill the machine and K is long.
     int64_t gemm_k_chunks(const gemm_request& request);

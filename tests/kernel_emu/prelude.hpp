@@ -12,7 +12,8 @@
 // wave's threads: on the GPU a wave's lanes run together and only the
 // compiler's ordering is at stake), wave64 __shfl_xor, __shfl, __ballot,
 // DPP row patterns,
-// v_mfma_f32_32x32x2f32 and v_mfma_f32_16x16x4f32 (barriers
+// v_mfma_f32_32x32x2f32, v_mfma_f32_16x16x4f32 and
+// v_mfma_f32_32x32x16_bf16 (barriers
 // over the wave's 64 threads, operand layouts as on gfx950), raw buffer
 // stores (range-checked against the resource's size), LDS arrays
 // (function-local statics, shared by the block's threads; blocks run one
@@ -143,6 +144,35 @@ namespace emu {
         return out;
     }
 
+    typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+    inline float wave_a8[16][64][8];
+    inline float wave_b8[16][64][8];
+
+    // v_mfma_f32_32x32x16_bf16: lane l holds A[l % 32][8 (l / 32) ..+7] and
+    // B[8 (l / 32) ..+7][l % 32]; accumulators as for 32x32x2f32.  The
+    // products are exact in fp32; here they are summed in double.
+    inline v16 mfma_32x32x16(b8 a, b8 b, v16 c) {
+        const int w = wave();
+        const int l = lane();
+        for (int e = 0; e < 8; ++e) {
+            wave_a8[w][l][e] = static_cast<float>(a[e]);
+            wave_b8[w][l][e] = static_cast<float>(b[e]);
+        }
+        wave_barrier[w]->arrive_and_wait();
+        v16 out = c;
+        for (int v = 0; v < 16; ++v) {
+            const int i = 8 * (v / 4) + 4 * (l / 32) + v % 4;
+            const int j = l % 32;
+            double sum = c[v];
+            for (int h = 0; h < 2; ++h)
+                for (int e = 0; e < 8; ++e)
+                    sum += static_cast<double>(wave_a8[w][i + 32 * h][e]) * wave_b8[w][j + 32 * h][e];
+            out[v] = static_cast<float>(sum);
+        }
+        wave_barrier[w]->arrive_and_wait();
+        return out;
+    }
+
     // A raw buffer resource (stride 0): stores at byte offsets at or past
     // num_records are dropped, as the hardware's range check does.
     struct buffer_rsrc {
@@ -182,11 +212,23 @@ namespace emu {
 #define __hip_atomic_load(p, order, scope) __atomic_load_n((p), (order))
 #define __hip_atomic_store(p, v, order, scope) __atomic_store_n((p), (v), (order))
 #define __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, x, y, z) emu::mfma_32x32x2((a), (b), (c))
+#define __builtin_amdgcn_iglp_opt(a) ((void)0)
+#define __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, x, y, z) emu::mfma_32x32x16((a), (b), (c))
 #define __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, x, y, z) emu::mfma_16x16x4((a), (b), (c))
 #define __builtin_amdgcn_update_dpp(old, src, ctrl, rm, bm, bc) emu::update_dpp((src), (ctrl))
 #define __builtin_amdgcn_make_buffer_rsrc(p, stride, num, flags) \
     emu::buffer_rsrc{reinterpret_cast<char*>(p), static_cast<uint32_t>(num)}
 #define __builtin_amdgcn_raw_buffer_store_b32(v, r, off, soff, aux) emu::buffer_store_b32((v), (r), (off) + (soff))
+
+// float to bf16, round to nearest even (clang's library call for the
+// conversion on a host without it)
+extern "C" inline __attribute__((used)) __bf16 __truncsfbf2(float x) {
+    unsigned u = __builtin_bit_cast(unsigned, x);
+    if (x != x) u |= 0x400000u;
+    else u += 0x7fffu + ((u >> 16) & 1u);
+    const unsigned short h = static_cast<unsigned short>(u >> 16);
+    return __builtin_bit_cast(__bf16, h);
+}
 
 struct __attribute__((aligned(16))) float4 {
     float x, y, z, w;

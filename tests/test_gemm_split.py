@@ -1,0 +1,167 @@
+"""fp32 products on the bf16 matrix cores (three bf16 values per fp32 one):
+tile edges, partial steps of K, operand layouts, both tile sizes, split K,
+and the values that the split cannot hold (recomputed with fp32 MFMAs)."""
+
+import numpy as np
+import pytest
+
+import porch_amd as porch
+from oracle import host
+from tests.helpers import placeholder
+from tests.kernel_emu import emulate as emu
+
+T = porch.transpose
+
+
+def ints(shape, rng):
+    return rng.integers(-8, 9, size=shape).astype(np.float32)
+
+
+def strided(x, rows, cols):
+    # every second row and column of a larger matrix: contiguous along neither
+    return x[porch.slice(0, 2 * rows, 2), porch.slice(1, 2 * cols + 1, 2)]
+
+
+# name: (shapes of A, B; graph).  K = 65 .. 130 covers partial steps of 1 to
+# 31 values (steps of 32) and none; extents around the 128-row tile, odd ones
+# for the two-row loads along the rows.
+SMALL = {
+    "one row past a tile": ([129, 66], [66, 130], lambda a, b: porch.matmul(a, b)),
+    "odd columns, epilogue": ([127, 97], [97, 129], lambda a, b: porch.relu(porch.matmul(a, b) - 3.0) * 0.5),
+    "both transposed, odd": ([65, 131], [67, 65], lambda a, b: porch.matmul(T(a), T(b))),
+    "transposed A, whole steps": ([96, 130], [96, 34], lambda a, b: porch.matmul(T(a), b)),
+    "strided operands": ([140, 141], [142, 261], lambda a, b: porch.matmul(strided(a, 70, 70), strided(b, 70, 130))),
+    "one column": ([2050, 130], [130, 1], lambda a, b: porch.batched_matmul(
+        porch.reshape(a, [1, 2050, 130]), porch.reshape(b, [1, 130, 1]))),
+    "batched, shared right side": ([3, 70, 100], [100, 35], lambda a, b: porch.batched_matmul(
+        a, porch.broadcast_to(b, [3, 100, 35]))),
+    "split K, partial step": ([40, 1030], [1030, 37], lambda a, b: porch.matmul(a, b) + 1.0),
+}
+
+
+def build(name, make):
+    sa, sb, f = SMALL[name]
+    return f(make(sa), make(sb))
+
+
+def filled(shape, values):
+    t = placeholder(shape)
+    t._state.storage = porch._Storage(None, np.ascontiguousarray(values, np.float32).reshape(-1))
+    return t
+
+
+@pytest.mark.skipif(not emu.available(), reason="no clang for the emulation")
+@pytest.mark.parametrize("name", ["both transposed, odd", "strided operands"])
+def test_emulated_products_bit_exact(name):
+    rng = np.random.default_rng(1)
+    sa, sb, f = SMALL[name]
+    a, b = ints(sa, rng), ints(sb, rng)
+    expr = f(filled(sa, a), filled(sb, b))
+    assert [k["kind"] for k in porch.plan(expr)["kernels"]] == ["gemm.mfma"]
+    assert all(r["ok"] for r in emu.emulate(expr, timeout=300))
+    got = emu.evaluate(expr, [a, b], timeout=300)
+    assert np.array_equal(got, host.evaluate(expr).reshape(got.shape))
+
+
+@pytest.mark.skipif(not emu.available(), reason="no clang for the emulation")
+def test_emulated_large_tiles_at_the_edges():
+    # 256 x 256 tiles (16 x 16 of them), a partial step of 3, ragged edges
+    rng = np.random.default_rng(2)
+    m, k, n = 3901, 67, 3999
+    a, b = ints((m, k), rng), ints((k, n), rng)
+    expr = porch.matmul(filled([m, k], a), filled([k, n], b))
+    (kernel,) = porch.plan(expr)["kernels"]
+    assert kernel["grid"][0] == 256
+    assert emu.check_edges(expr, [a, b], host.evaluate(expr).reshape(m, n)) > 4 * 150 * 150
+
+
+# Operand values past what three bf16 values hold, planted into A: the
+# results are the fp32 MFMA's, in the oracle's (sequential) order here.
+SPECIAL = {
+    "infinity": [np.inf], "both infinities": [np.inf, -np.inf], "nan": [np.nan],
+    "largest": [3.4028235e38], "rounds up to an infinite bf16": [-3.4e38],
+    "denormal": [1e-40], "least denormal": [1.4e-45], "below 2^-109": [1.5e-33 * 0.9],
+}
+
+
+def special_inputs(name, m, k, n):
+    rng = np.random.default_rng(3)
+    a = rng.uniform(0.5, 2.0, size=(m, k)).astype(np.float32)
+    b = rng.uniform(0.5, 2.0, size=(k, n)).astype(np.float32)
+    a[1] = 0.0  # a row of its own: nothing hides the value
+    for i, x in enumerate(SPECIAL[name]):
+        a[1, 3 + i] = np.float32(x)
+        a[2, 5 + i] = np.float32(x)
+        if abs(x) > 1e30:
+            b[3 + i] = 2.0 ** -20
+        elif abs(x) < 1e-30:
+            b[3 + i] = 2.0 ** 100
+            b[3 + i, : n // 2] = 3.0
+    return a, b
+
+
+def check_special(got, a, b, want):
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    fin = np.isfinite(want)
+    assert np.array_equal(got[~fin & ~np.isnan(want)], want[~fin & ~np.isnan(want)])
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    with np.errstate(invalid="ignore", over="ignore"):
+        exact, scale = a64 @ b64, np.abs(a64) @ np.abs(b64)
+    # K roundings of fp32, or half the least denormal where that is more
+    assert np.all(np.abs(got[fin] - exact[fin]) <= (a.shape[1] * 2.0 ** -24 * scale)[fin] + 2.0 ** -150)
+
+
+@pytest.mark.skipif(not emu.available(), reason="no clang for the emulation")
+@pytest.mark.parametrize("name", ["both infinities", "least denormal"])
+def test_emulated_special_values(name):
+    m, k, n = 40, 96, 72
+    a, b = special_inputs(name, m, k, n)
+    expr = porch.matmul(filled([m, k], a), filled([k, n], b))
+    got = emu.evaluate(expr, [a, b], timeout=300)
+    check_special(got.reshape(m, n), a, b, host.evaluate(expr).reshape(m, n))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", sorted(SMALL))
+def test_products_bit_exact_on_integers(gpu, name):
+    rng = np.random.default_rng(4)
+    expr = build(name, lambda s: gpu.tensor(s, ints(s, rng).reshape(-1)))
+    out = gpu.materialize(expr).cpu().reshape(expr.shape())
+    assert np.array_equal(out, host.evaluate(expr).reshape(out.shape))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m, k, n, ta, tb", [(3901, 67, 3999, False, False), (3901, 80, 3999, True, True)])
+def test_large_tiles_bit_exact_on_integers(gpu, m, k, n, ta, tb):
+    rng = np.random.default_rng(5)
+    a, b = ints((k, m) if ta else (m, k), rng), ints((n, k) if tb else (k, n), rng)
+    x, y = gpu.tensor(list(a.shape), a.reshape(-1)), gpu.tensor(list(b.shape), b.reshape(-1))
+    expr = porch.matmul(T(x) if ta else x, T(y) if tb else y)
+    assert gpu.plan(expr)["kernels"][0]["grid"][0] == 256
+    out = gpu.materialize(expr).cpu().reshape(m, n)
+    want = (a.T if ta else a).astype(np.float64) @ (b.T if tb else b).astype(np.float64)
+    assert np.array_equal(out, want.astype(np.float32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", sorted(SPECIAL))
+def test_special_values(gpu, name):
+    for m, k, n in [(200, 96, 300), (130, 1100, 150)]:
+        a, b = special_inputs(name, m, k, n)
+        expr = porch.matmul(gpu.tensor([m, k], a.reshape(-1)), gpu.tensor([k, n], b.reshape(-1)))
+        out = gpu.materialize(expr).cpu().reshape(m, n)
+        check_special(out, a, b, host.evaluate(expr).reshape(m, n))
+
+
+@pytest.mark.gpu
+def test_tiny_values_beside_ordinary_results(gpu):
+    # values below 2^-109 in a product whose results are all 2^-56 and more:
+    # the split's own results, within K roundings of fp32
+    rng = np.random.default_rng(6)
+    m, k, n = 300, 200, 260
+    a = rng.uniform(0.5, 1.0, size=(m, k)).astype(np.float32)
+    a[:, 7] = 1e-38
+    b = rng.uniform(0.5, 1.0, size=(k, n)).astype(np.float32)
+    out = gpu.materialize(porch.matmul(gpu.tensor([m, k], a.reshape(-1)), gpu.tensor([k, n], b.reshape(-1))))
+    exact = a.astype(np.float64) @ b.astype(np.float64)
+    assert np.all(np.abs(out.cpu().reshape(m, n) - exact) <= k * 2.0 ** -24 * exact)
