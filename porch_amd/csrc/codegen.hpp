@@ -25,8 +25,12 @@
 //                    axis with lanes along the contiguous output dimension;
 //   reduce.column_softmax  the same layout folding a softmax's max and sum
 //                    (relative to a moving anchor) in one read;
-//   gemm             LDS-tiled v_mfma_f32_32x32x2f32 with the elementwise
-//                    epilogue applied to the accumulators before the store;
+//   gemm.mfma        products on the matrix cores: three bf16 values per fp32
+//                    one, or for many tiles of a short K persistent
+//                    workgroups on fp32 MFMAs, the elementwise epilogue
+//                    applied to the accumulators before the store;
+//   attention        softmax of a product along its last axis, times a third
+//                    matrix, without the scores in memory;
 //   gemm.rows,       products with a few rows (or columns), streaming the
 //   gemm.cols        long operand once;
 //   gemm.narrow      7 to 32 columns over many rows: v_mfma_f32_16x16x4f32
@@ -166,6 +170,10 @@ namespace porch::cg {
         int64_t stride_row = 0;   // A: per m, B: per k
         int64_t stride_col = 0;   // A: per k, B: per n
         int64_t stride_batch = 0; // per batch entry (0: shared)
+        // > 0: entries in groups of this many, stride_batch apart within a
+        // group, stride_batch_outer from group to group (attention only)
+        int64_t batch_inner = 0;
+        int64_t stride_batch_outer = 0;
     };
     struct gemm_request {
         const kexpr* expr = nullptr;
@@ -221,6 +229,27 @@ namespace porch::cg {
     bool gemm_wide(const gemm_request& request);
     int64_t gemm_wide_chunks(const gemm_request& request);
     kernel_code emit_gemm_wide(const gemm_request& request);
+
+    // softmax(f(Q K), last axis) V in one kernel (emit_attention.cpp).
+    struct attention_request {
+        bool batched = false;
+        int64_t batch = 1;
+        int64_t rows = 0, keys = 0; // of the scores
+        int64_t dim = 0;            // of Q's rows and of V's
+        gemm_operand q;             // per query, per dim
+        gemm_operand k;             // per dim, per key (the product's right side)
+        gemm_operand v;             // per key, per dim
+        const kexpr* score_expr = nullptr;
+        int score = -1;             // f over (b, query, key); row_value 0: the product
+        const kexpr* expr = nullptr;
+        int epilogue = -1;          // over (b, query, dim); row_value 0: the result
+        int n_slots = 0;
+        index_width width;
+        int compute_units = 256;
+    };
+    // dim of 32, 64 or 128, 32 rows and keys or more.
+    bool attention_fits(int64_t rows, int64_t keys, int64_t dim, int64_t value_dim);
+    kernel_code emit_attention(const attention_request& request);
 
     // A short K (8 to 64, a multiple of 8) over 256 columns or more, A's
     // rows contiguous along K and B's rows along N or its columns along K

@@ -1,0 +1,528 @@
+// softmax(f(Q K), last axis) V in one kernel: the scores never reach memory.
+//
+// Unfused, the product of 16 heads over 4096 positions writes 1 GiB of
+// scores, the softmax reads and writes them and the second product reads
+// them again: 1186 us with both products on the matrix cores, most of it
+// those 4 GiB.  Here a wave owns 32 queries and walks the keys in tiles; per
+// tile it computes S^T = K Q^T, the running row maximum m, p = exp(s - m),
+// and adds V^T P^T to its output, rescaling output and row sum whenever the
+// maximum grows, and divides by the sum at the end.
+//
+// Both products run on the bf16 MFMA over fp32 values split into three bf16
+// values (see emit_gemm_split.cpp for the split, its error and its limits).
+// The transposed products put a query in a lane: the 32 x 32 x 16 MFMA gives
+// lane l the scores of query l % 32 for keys 8 g + 4 (l / 32) + (0 .. 3), and
+// wants the same lane's eight values per 16 keys as its operand of the second
+// product.  The order of keys inside a product is free, so the tile of V is
+// stored in the order the lane already holds and P never leaves its
+// registers; a row's maximum and sum need one exchange between the lane's
+// two halves of the wave.
+//
+// An iteration computes the products of the next tile, the weights of this
+// one and the sums of the one before: independent of each other, so that a
+// wave's MFMAs run beside its exps and splits (up to six vector instructions
+// fit beside one 32-cycle MFMA).
+//
+// What bounds it: the bf16 MFMAs at the rate the card sustains.  2 x 8 heads
+// of 4096 positions, dim 64: 342 us and 8 us for the permute behind it (1438
+// us unfused on fp32 MFMAs, 1186 with both products on bf16 ones); the six
+// products of the split make that 1.2 PFLOP/s of bf16, against the 1.34-1.42
+// that this card's large bf16 products reach.
+//
+// Accuracy: a weight is exp2(s log2 e - M) with M the running maximum of
+// s log2 e: one rounding, and whatever M's own rounding is cancels against
+// the row's sum.  Weights reach the second product in 24 bits relative to the
+// row's maximum down to 2^-109 of it (smaller ones lose at most 2^-133).
+// Against 64 bits, normal q, k and v: 1.0e-6 (the unfused program: 1.2e-6).
+// What this cannot hold (values that are not finite anywhere, nonzero Q or K
+// below 2^-109, nonzero V below 2^-109 beside an output below 2^-56 or
+// operands of 2^30, rows whose scores are all below -2^100) sends the
+// workgroup to `redo`: fp32 MFMAs, in the unfused program's order.
+
+#include "emit_gemm.hpp"
+
+#include <algorithm>
+#include <stdexcept>
+
+namespace porch::cg {
+
+    namespace {
+
+        // A tile of K (rows: keys) or V^T (rows: dims) and how it is read:
+        // along its inner side (k: dims of K, keys of V), 128 bits of a row;
+        // along its rows, four loads of two rows; or value by value.
+        enum class reading { along_k, along_rows, strided };
+
+        struct tile_operand {
+            std::string x;      // "K" or "V"
+            bool keys_in_rows;  // K: rows are keys; V: the inner side is
+            int rows, inner;
+            int64_t stride_row, stride_k;
+            reading how;
+            int units, values;
+        };
+
+        tile_operand tile_of(const std::string& x, bool keys_in_rows, int rows, int inner, int64_t stride_row,
+                             int64_t stride_k, int threads) {
+            tile_operand o{x, keys_in_rows, rows, inner, stride_row, stride_k, reading::strided, 0, 4};
+            if (stride_k == 1) o.how = reading::along_k;
+            else if (stride_row == 1) o.how = reading::along_rows;
+            o.values = o.how == reading::along_rows && rows * inner / 8 >= threads ? 8 : 4;
+            o.units = rows * inner / o.values / threads;
+            return o;
+        }
+
+        // LDS holds [slice of 16][octet][row][h, m, l of 8 values], 48 bytes a
+        // row.  Rows of octet o sit at row ^ x(o), so that the octets of a row
+        // that adjacent lanes write meet different banks.
+        int swizzle_of(const tile_operand& o) { return 128 / o.inner; }
+
+        std::string setup_code(const tile_operand& o, int threads, const char* offset_type) {
+            std::string s;
+            const std::string OT = offset_type, R = std::to_string(o.rows), X = std::to_string(swizzle_of(o));
+            for (int i = 0; i < o.units; ++i) {
+                const std::string id = o.x + std::to_string(i);
+                s += "    const int c" + id + " = tid + " + std::to_string(i * threads) + ";\n";
+                std::string row;
+                if (o.how == reading::along_rows) {
+                    // adjacent lanes write adjacent LDS rows
+                    const std::string across = std::to_string(o.rows * 4 / o.values);
+                    s += "    const int oct" + id + " = (c" + id + " >> 1) / " + across + ";\n";
+                    s += "    const int half" + id + " = c" + id + " & 1;\n";
+                    const std::string at = "((c" + id + " >> 1) % " + across + ")";
+                    s += "    const int i" + id + " = " +
+                         (o.values == 8 ? at + " * 2" : o.keys_in_rows ? at : "porch_row_dim(" + at + ")") + ";\n";
+                    // V's key order: octet h holds keys 4 h .. and 8 + 4 h ..
+                    s += "    const int kq" + id + " = " +
+                         (o.keys_in_rows ? "oct" + id + " * 8 + half" + id + " * 4"
+                                         : "(oct" + id + " >> 1) * 16 + half" + id + " * 8 + (oct" + id + " & 1) * 4") +
+                         ";\n";
+                }
+                else {
+                    const std::string per_row = std::to_string(o.inner / 4);
+                    s += "    const int kq" + id + " = (c" + id + " % " + per_row + ") * 4;\n";
+                    s += "    const int i" + id + " = c" + id + " / " + per_row + ";\n";
+                    s += "    const int oct" + id + " = " +
+                         (o.keys_in_rows ? "kq" + id + " >> 3"
+                                         : "(kq" + id + " >> 4) * 2 + ((kq" + id + " >> 2) & 1)") +
+                         ";\n";
+                    s += "    const int half" + id + " = (kq" + id + " >> " + (o.keys_in_rows ? "2" : "3") + ") & 1;\n";
+                }
+                s += "    const " + OT + " o" + id + " = ((" + OT + ")i" + id + " * " + std::to_string(o.stride_row) + " + (" +
+                     OT + ")kq" + id + " * " + std::to_string(o.stride_k) + ") * 4;\n";
+                for (int e = 0; e < o.values / 4; ++e) {
+                    const std::string at = "(i" + id + " + " + std::to_string(e) + ")";
+                    s += "    const int w" + id + (e ? "b" : "") + " = (oct" + id + " * " + R + " + (" +
+                         (o.keys_in_rows ? at : "porch_dim_row" + at) + " ^ (oct" + id + " * " + X + "))) * 12 + half" +
+                         id + " * 2;\n";
+                }
+            }
+            s += "    float r" + o.x + "[" + std::to_string(o.units * o.values) + "];\n";
+            return s;
+        }
+
+        // The tile whose first key is `key0` into registers; `valid` (empty:
+        // all): only keys below it exist, the rest read as zero.
+        std::string load_code(const tile_operand& o, const std::string& key0, const std::string& valid,
+                              const std::string& ind) {
+            const std::string stride = std::to_string(o.keys_in_rows ? o.stride_row : o.stride_k);
+            std::string s = ind + "{\n" + ind + "    const char* __restrict__ base = (const char*)(" + o.x + " + (idx_t)(" +
+                            key0 + ") * " + stride + ");\n";
+            for (int i = 0; i < o.units; ++i) {
+                const std::string id = o.x + std::to_string(i);
+                auto reg = [&](int j) { return "r" + o.x + "[" + std::to_string(i * o.values + j) + "]"; };
+                if (o.how == reading::along_k && (valid.empty() || o.keys_in_rows)) {
+                    s += ind + "    porch_f4u v" + id + " = {0.0f, 0.0f, 0.0f, 0.0f};\n";
+                    s += ind + "    " + (valid.empty() ? std::string() : "if (i" + id + " < " + valid + ") ") + "v" + id +
+                         " = *(const porch_f4u*)(base + o" + id + ");\n" + ind + "    ";
+                    const char* e[] = {"x", "y", "z", "w"};
+                    for (int j = 0; j < 4; ++j) s += reg(j) + " = v" + id + "." + e[j] + "; ";
+                    s += "\n";
+                    continue;
+                }
+                for (int j = 0; j < 4; ++j) {
+                    const std::string J = std::to_string(j);
+                    const std::string p = "base + o" + id + " + " + std::to_string(j * o.stride_k * 4) + "LL";
+                    if (o.values == 8 && (valid.empty() || !o.keys_in_rows)) {
+                        s += ind + "    porch_f2u v" + id + J + " = {0.0f, 0.0f};\n";
+                        s += ind + "    " + (valid.empty() ? std::string() : "if (kq" + id + " + " + J + " < " + valid + ") ") +
+                             "v" + id + J + " = *(const porch_f2u*)(" + p + ");\n";
+                        s += ind + "    " + reg(j) + " = v" + id + J + ".x; " + reg(4 + j) + " = v" + id + J + ".y;\n";
+                        continue;
+                    }
+                    for (int e = 0; e < o.values / 4; ++e) {
+                        const std::string key = o.keys_in_rows ? "i" + id + " + " + std::to_string(e) : "kq" + id + " + " + J;
+                        s += ind + "    " + reg(4 * e + j) + " = " + (valid.empty() ? std::string() : key + " < " + valid + " ? ") +
+                             "*(const float*)(" + p + " + " + std::to_string(e * 4) + ")" + (valid.empty() ? "" : " : 0.0f") +
+                             ";\n";
+                    }
+                }
+            }
+            return s + ind + "}\n";
+        }
+
+        std::string store_code(const tile_operand& o, const std::string& buffer, const std::string& ind) {
+            std::string s;
+            for (int i = 0; i < o.units; ++i)
+                for (int e = 0; e < o.values / 4; ++e) {
+                    s += ind + "porch_split4(";
+                    for (int j = 0; j < 4; ++j) s += "r" + o.x + "[" + std::to_string(i * o.values + 4 * e + j) + "], ";
+                    s += "&" + o.x + "s[" + buffer + "][0][0][0] + w" + o.x + std::to_string(i) + (e ? "b" : "") + ", lowest" +
+                         o.x + ", largest);\n";
+                }
+            return s;
+        }
+
+        // Can four scores of adjacent keys be emitted together: every input
+        // of f at an affine index, no branches.
+        bool vector_scores(const kexpr& k, int root) {
+            for (const int id : k.postorder(root)) {
+                const knode& n = k.at(id);
+                if (n.op == kop::select) return false;
+                if (n.op == kop::load && !n.index.is_affine) return false;
+            }
+            return true;
+        }
+
+        const char* helpers() {
+            return R"(typedef unsigned porch_u4 __attribute__((ext_vector_type(4)));
+// LDS row of dim d of V^T: pairs of adjacent dims lie 16 apart.
+__device__ __forceinline__ int porch_dim_row(int d) { return (d & ~31) | ((d & 1) << 4) | ((d >> 1) & 15); }
+__device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 15) << 1) | ((p >> 4) & 1); }
+)";
+        }
+
+    } // namespace
+
+    bool attention_fits(int64_t rows, int64_t keys, int64_t dim, int64_t value_dim) {
+        return dim == value_dim && (dim == 32 || dim == 64 || dim == 128) && rows >= 32 && keys >= 32;
+    }
+
+    kernel_code emit_attention(const attention_request& r) {
+        if (!attention_fits(r.rows, r.keys, r.dim, r.dim)) throw std::logic_error("emit_attention: shape");
+        const int D = static_cast<int>(r.dim);
+        // keys a tile: two buffers of K and V in 48 KB of LDS (96 at dim 128)
+        const int KT = std::max(32, 2048 / D);
+        const int KB = KT / 32, DB = D / 32, DS = D / 16;
+        // Eight waves (256 queries) a workgroup share each tile of K and V;
+        // four where that still leaves no compute unit a second workgroup.
+        const int64_t cus = std::max(r.compute_units, 8);
+        const int waves = r.batch * ((r.rows + 127) / 128) <= cus ? 4 : 8;
+        const int threads = 64 * waves;
+        const int BQ = 32 * waves;
+        const int64_t tiles = (r.rows + BQ - 1) / BQ;
+        const int64_t total = tiles * r.batch;
+        const int64_t full = r.keys / KT, tail = r.keys % KT;
+        const int64_t steps = full + (tail != 0 ? 1 : 0);
+        const std::string SQ = std::to_string(r.rows), SK = std::to_string(r.keys), DD = std::to_string(D);
+        const std::string KTS = std::to_string(KT), KBS = std::to_string(KB), DBS = std::to_string(DB), DSS = std::to_string(DS);
+        const char* OT = r.width.wide ? "long long" : "unsigned";
+        const tile_operand K = tile_of("K", true, KT, D, r.k.stride_col, r.k.stride_row, threads);
+        const tile_operand V = tile_of("V", false, D, KT, r.v.stride_col, r.v.stride_row, threads);
+
+        kernel_code kc;
+        kc.kind = "attention";
+        kc.name = "porch_attention";
+        kc.n_slots = r.n_slots;
+        kc.block = static_cast<unsigned>(threads);
+        kc.grid_x = static_cast<unsigned>(total);
+        std::string& s = kc.source;
+        s = kernel_prologue(r.n_slots, r.width.type());
+        s += bf16_split_helpers();
+        s += helpers();
+        s += "extern \"C\" __global__ void __launch_bounds__(" + std::to_string(threads) + ", " + (waves == 8 ? "2" : "1") +
+             ") porch_attention(" + kernel_params(r.n_slots) + ") {\n";
+        s += "    __shared__ __attribute__((aligned(16))) float Ks[2][" + DSS + "][" + std::to_string(2 * KT) + "][12];\n";
+        s += "    __shared__ __attribute__((aligned(16))) float Vs[2][" + std::to_string(KT / 16) + "][" +
+             std::to_string(2 * D) + "][12];\n";
+        s += "    __shared__ unsigned seen[8];\n";
+        s += "    const int tid = threadIdx.x;\n    const int lane = tid & 63;\n    const int wave = tid >> 6;\n";
+        s += "    const int h = lane >> 5;\n";
+        // an XCD takes whole heads where it can: its L2 holds their K and V
+        const int64_t each = total / 8, more = total % 8;
+        s += "    const int xcd = blockIdx.x % 8;\n";
+        s += "    const idx_t lin = (idx_t)xcd * " + std::to_string(each) +
+             (more ? " + (xcd < " + std::to_string(more) + " ? xcd : " + std::to_string(more) + ")" : std::string()) +
+             " + blockIdx.x / 8;\n";
+        if (r.batched) s += "    const idx_t qb = lin / " + std::to_string(tiles) + ";\n";
+        s += "    const idx_t own = (lin" + (r.batched ? " % " + std::to_string(tiles) : std::string()) + ") * " +
+             std::to_string(BQ) + " + wave * 32 + (lane & 31);\n";
+        s += "    const idx_t q0 = own < " + SQ + " ? own : (idx_t)" + SQ + " - 1;\n";
+        auto base = [&](const char* x, const gemm_operand& op) {
+            s += std::string("    const float* __restrict__ ") + x + " = a" + std::to_string(op.slot) + " + " +
+                 std::to_string(op.offset);
+            if (r.batched && op.batch_inner > 0)
+                s += " + qb / " + std::to_string(op.batch_inner) + " * " + std::to_string(op.stride_batch_outer) +
+                     " + qb % " + std::to_string(op.batch_inner) + " * " + std::to_string(op.stride_batch);
+            else if (r.batched && op.stride_batch != 0)
+                s += " + qb * " + std::to_string(op.stride_batch);
+            s += ";\n";
+        };
+        base("Q", r.q);
+        base("K", r.k);
+        base("V", r.v);
+        s += setup_code(K, threads, OT) + setup_code(V, threads, OT);
+        s += "    unsigned lowestK = 0xffffffffu, lowestV = 0xffffffffu;\n    porch_s2 largest = {0, 0};\n";
+        const std::string partial = std::to_string(full * KT);
+        const std::string ahead_of = tail != 0 ? " - 1" : "";
+        auto whole = [&](const std::string& g) { return "(" + g + ahead_of + ") * " + KTS; };
+        // the partial tile first, so that the loop's loads need no tests
+        const std::string valid = tail != 0 ? std::to_string(tail) : "";
+        s += load_code(K, tail != 0 ? partial : "0", valid, "    ") + load_code(V, tail != 0 ? partial : "0", valid, "    ");
+        // this lane's query, split
+        s += "    porch_b8 qf[" + DSS + "][3];\n";
+        s += "    #pragma unroll\n    for (int t = 0; t < " + DSS + "; ++t) {\n        porch_u4 u[3];\n";
+        s += "        #pragma unroll\n        for (int e = 0; e < 4; ++e) {\n";
+        s += "            const idx_t at = q0 * " + std::to_string(r.q.stride_row) + " + (idx_t)(t * 16 + h * 8 + 2 * e) * " +
+             std::to_string(r.q.stride_col) + ";\n            unsigned x, y, z;\n";
+        s += "            porch_split2(Q[at], Q[at + " + std::to_string(r.q.stride_col) + "], x, y, z, lowestK, largest);\n";
+        s += "            u[0][e] = x; u[1][e] = y; u[2][e] = z;\n        }\n";
+        s += "        #pragma unroll\n        for (int p = 0; p < 3; ++p) qf[t][p] = __builtin_bit_cast(porch_b8, u[p]);\n    }\n";
+        s += store_code(K, "0", "    ");
+        if (steps > 1) {
+            s += load_code(K, whole("1"), "", "    ") + store_code(K, "1", "    ");
+            s += load_code(K, whole(steps > 2 ? "2" : "1"), "", "    ");
+        }
+        s += "    float m = -0x1p100f, sum = 0.0f, top = 0.0f;\n    porch_v16f acc[" + DBS + "], sc[" + KBS + "];\n    porch_b8 pf[" + std::to_string(KT / 16) + "][3];\n";
+        const std::string zero_acc = "    #pragma unroll\n    for (int d = 0; d < " + DBS +
+                                     "; ++d)\n        #pragma unroll\n        for (int v = 0; v < 16; ++v) acc[d][v] = 0.0f;\n";
+        s += zero_acc + "    __syncthreads();\n";
+
+        // f of the 16 products sc[kb][..] of keys key0 + kb 32 + 8 g + 4 h + j
+        const bool vec = vector_scores(*r.score_expr, r.score);
+        auto scores = [&](const std::string& sc, const std::string& key, bool masked, const std::string& ind) {
+            std::string c = ind + "#pragma unroll\n" + ind + "for (int g = 0; g < 4; ++g) {\n";
+            c += ind + "    const idx_t key = " + key + " + 8 * g + 4 * h;\n" + ind + "    (void)key;\n";
+            auto names = [&](const std::string& q1) {
+                return r.batched ? std::vector<std::string>{"qb", "q0", q1} : std::vector<std::string>{"q0", q1};
+            };
+            if (vec && !masked) {
+                std::string body;
+                emitter em(*r.score_expr, body, 4);
+                em.indent = ind + "    ";
+                em.declare_roots({r.score});
+                em.load = [&](int id) {
+                    const knode& n = r.score_expr->at(id);
+                    const std::string at = "a" + std::to_string(n.slot);
+                    const int64_t w = n.index.w.back();
+                    const std::string ix = index_text(n.index, names("key"));
+                    if (w == 0) return std::vector<std::string>(4, at + "[" + ix + "]");
+                    if (w == 1) {
+                        const std::string f = em.fresh("f");
+                        em.line("const porch_f4u " + f + " = *(const porch_f4u*)&" + at + "[" + ix + "];");
+                        return std::vector<std::string>{f + ".x", f + ".y", f + ".z", f + ".w"};
+                    }
+                    std::vector<std::string> v;
+                    for (int j = 0; j < 4; ++j) v.push_back(at + "[" + ix + " + " + std::to_string(j * w) + "]");
+                    return v;
+                };
+                em.row_value = [](int) { return std::string("porch_lane_product"); };
+                em.override_node = [&](int id) {
+                    if (r.score_expr->at(id).op != kop::row_value) return std::vector<std::string>{};
+                    std::vector<std::string> v;
+                    for (int j = 0; j < 4; ++j) v.push_back(sc + "[4 * g + " + std::to_string(j) + "]");
+                    return v;
+                };
+                const std::vector<std::string> v = em.emit(r.score);
+                c += body;
+                for (int j = 0; j < 4; ++j) c += ind + "    const float x" + std::to_string(j) + " = " + v[static_cast<size_t>(j)] + ";\n";
+                for (int j = 0; j < 4; ++j) c += ind + "    " + sc + "[4 * g + " + std::to_string(j) + "] = x" + std::to_string(j) + ";\n";
+            }
+            else {
+                gemm_request e;
+                e.expr = r.score_expr;
+                e.epilogue = r.score;
+                c += ind + "    #pragma unroll\n" + ind + "    for (int j = 0; j < 4; ++j) {\n";
+                c += ind + "        const idx_t q1 = key + j" + (masked ? " < " + SK + " ? key + j : (idx_t)" + SK + " - 1" : std::string()) + ";\n";
+                c += ind + "        (void)q1;\n" + ind + "        const float acc_v = " + sc + "[4 * g + j];\n";
+                std::string body;
+                emitter em(*r.score_expr, body, 1);
+                em.indent = ind + "        ";
+                em.declare_roots({r.score});
+                epilogue_emitter(em, e, names("q1"), "acc_v");
+                const std::string v = em.emit(r.score)[0];
+                c += body + ind + "        " + sc + "[4 * g + j] = " +
+                     (masked ? "key + j < " + SK + " ? " + v + " : -__builtin_inff()" : v) + ";\n" + ind + "    }\n";
+            }
+            return c + ind + "}\n";
+        };
+
+        // One wave a SIMD hides its own latencies: an MFMA, an LDS read,
+        // five vector instructions, and so on (8 heads of 2048 positions,
+        // dim 64: 102 us against 128 in the compiler's order).  With two
+        // waves a SIMD, or the longer products of dim 128, the compiler's
+        // order is the faster one (16 heads of 4096: 365 us against 392).
+        auto schedule = [&](const std::string& ind) {
+            std::string c;
+            if (waves != 4 || D == 128) return c;
+            c += ind + "__builtin_amdgcn_sched_group_barrier(0x100, 3, 0);\n";
+            for (int i = 0; i < 6 * DS * KB + 6 * (KT / 16) * DB; ++i) {
+                c += ind + "__builtin_amdgcn_sched_group_barrier(0x008, 1, 0);\n";
+                c += ind + "__builtin_amdgcn_sched_group_barrier(0x100, 1, 0);\n";
+                c += ind + "__builtin_amdgcn_sched_group_barrier(0x002, 5, 0);\n";
+            }
+            return c;
+        };
+        constexpr int pairs[6][2] = {{0, 0}, {1, 0}, {0, 1}, {1, 1}, {2, 0}, {0, 2}};
+        // S^T of one tile of keys from K's buffer `kb` into `sc`
+        auto products = [&](const std::string& sc, const std::string& kb, const std::string& ind) {
+            std::string c;
+            c += ind + "#pragma unroll\n" + ind + "for (int b = 0; b < " + KBS + "; ++b)\n" + ind +
+                 "    #pragma unroll\n" + ind + "    for (int v = 0; v < 16; ++v) " + sc + "[b][v] = 0.0f;\n";
+            c += ind + "#pragma unroll\n" + ind + "for (int t = 0; t < " + DSS + "; ++t) {\n";
+            c += ind + "    const int row = (lane & 31) ^ ((2 * t + h) * " + std::to_string(swizzle_of(K)) + ");\n";
+            c += ind + "    porch_b8 kf[" + KBS + "][3];\n";
+            c += ind + "    #pragma unroll\n" + ind + "    for (int b = 0; b < " + KBS + "; ++b)\n" + ind + "        #pragma unroll\n" +
+                 ind + "        for (int p = 0; p < 3; ++p) kf[b][p] = *(const porch_b8*)&Ks[" + kb + "][t][h * " + KTS +
+                 " + b * 32 + row][p * 4];\n";
+            for (const auto& pr : pairs)
+                c += ind + "    #pragma unroll\n" + ind + "    for (int b = 0; b < " + KBS + "; ++b) " + sc +
+                     "[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[b][" + std::to_string(pr[0]) + "], qf[t][" +
+                     std::to_string(pr[1]) + "], " + sc + "[b], 0, 0, 0);\n";
+            return c + ind + "}\n";
+        };
+        // the weights of the tile of scores in sc, split into pf, with the
+        // new maximum, the sum and the factor `alpha` for what came before
+        auto weights = [&](const std::string& key0, bool masked, const std::string& pf, const std::string& ind) {
+            std::string c;
+            c += ind + "#pragma unroll\n" + ind + "for (int b = 0; b < " + KBS + "; ++b) {\n";
+            c += ind + "    #pragma unroll\n" + ind + "    for (int v = 0; v < 16; ++v) top = __builtin_fmaxf(top, __builtin_fabsf(sc[b][v]));\n";
+            c += scores("sc[b]", "(idx_t)(" + key0 + ") + b * 32", masked, ind + "    ");
+            c += ind + "}\n";
+            c += ind + "float tm = sc[0][0];\n";
+            c += ind + "#pragma unroll\n" + ind + "for (int b = 0; b < " + KBS + "; ++b)\n" + ind + "    #pragma unroll\n" + ind +
+                 "    for (int v = 0; v < 16; ++v) tm = __builtin_fmaxf(tm, sc[b][v]);\n";
+            c += ind + "tm = __builtin_fmaxf(tm, __shfl_xor(tm, 32, 64));\n";
+            c += ind + "const float ml = __builtin_fmaxf(m, tm * 0x1.715476p+0f);\n";
+            c += ind + "const float alpha = __builtin_amdgcn_exp2f(m - ml);\n" + ind + "m = ml;\n";
+            c += ind + "float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};\n";
+            c += ind + "#pragma unroll\n" + ind + "for (int b = 0; b < " + KBS + "; ++b)\n" + ind + "    #pragma unroll\n" + ind +
+                 "    for (int v = 0; v < 16; ++v) {\n" + ind + "        sc[b][v] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[b][v], 0x1.715476p+0f, -m));\n" + ind +
+                 "        part[v & 3] += sc[b][v];\n" + ind + "    }\n";
+            c += ind + "sum = sum * alpha + ((part[0] + part[1]) + (part[2] + part[3]));\n";
+            c += ind + "#pragma unroll\n" + ind + "for (int t = 0; t < " + std::to_string(KT / 16) + "; ++t) {\n";
+            c += ind + "    porch_u4 u[3];\n" + ind + "    #pragma unroll\n" + ind + "    for (int e = 0; e < 4; ++e) {\n" + ind +
+                 "        unsigned x, y, z;\n" + ind +
+                 "        porch_split2(sc[t >> 1][(t & 1) * 8 + 2 * e], sc[t >> 1][(t & 1) * 8 + 2 * e + 1], x, y, z);\n" + ind +
+                 "        u[0][e] = x; u[1][e] = y; u[2][e] = z;\n" + ind + "    }\n";
+            c += ind + "    #pragma unroll\n" + ind + "    for (int p = 0; p < 3; ++p) " + pf +
+                 "[t][p] = __builtin_bit_cast(porch_b8, u[p]);\n" + ind + "}\n";
+            return c;
+        };
+        // acc += V^T P^T for the weights in pf and V's buffer `vb`
+        auto gather = [&](const std::string& vb, const std::string& ind) {
+            std::string c;
+            c += ind + "#pragma unroll\n" + ind + "for (int t = 0; t < " + std::to_string(KT / 16) + "; ++t) {\n";
+            c += ind + "    const int row = (lane & 31) ^ ((2 * t + h) * " + std::to_string(swizzle_of(V)) + ");\n";
+            c += ind + "    porch_b8 vf[" + DBS + "][3];\n";
+            c += ind + "    #pragma unroll\n" + ind + "    for (int d = 0; d < " + DBS + "; ++d)\n" + ind + "        #pragma unroll\n" +
+                 ind + "        for (int p = 0; p < 3; ++p) vf[d][p] = *(const porch_b8*)&Vs[" + vb + "][t][h * " + DD +
+                 " + d * 32 + row][p * 4];\n";
+            for (const auto& pr : pairs)
+                c += ind + "    #pragma unroll\n" + ind + "    for (int d = 0; d < " + DBS +
+                     "; ++d) acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[d][" + std::to_string(pr[0]) + "], pf[t][" +
+                     std::to_string(pr[1]) + "], acc[d], 0, 0, 0);\n";
+            return c + ind + "}\n";
+        };
+        // Iteration `it`: the products of tile it + 1, the weights of tile it
+        // and the sums of tile it - 1 are independent, so that one wave's MFMAs
+        // run beside its exps and splits; K is staged two tiles ahead, V
+        // with its weights.
+        auto iteration = [&](const std::string& key0, bool first, bool masked) {
+            std::string c;
+            const std::string ind = "        ";
+            c += ind + "porch_v16f sn[" + KBS + "];\n" + products("sn", "(it + 1) & 1", ind);
+            if (!first) c += gather("(it - 1) & 1", ind);
+            c += ind + "porch_b8 pn[" + std::to_string(KT / 16) + "][3];\n";
+            c += weights(key0, masked, "pn", ind);
+            if (steps > 1) c += store_code(K, "it & 1", ind);
+            c += store_code(V, "it & 1", ind);
+            if (steps > 1) {
+                c += ind + "const int ak = it + 3 < " + std::to_string(steps) + " ? it + 3 : " + std::to_string(steps - 1) + ";\n";
+                c += load_code(K, whole("ak"), "", ind);
+                c += ind + "const int av = it + 1 < " + std::to_string(steps) + " ? it + 1 : " + std::to_string(steps - 1) + ";\n";
+                c += load_code(V, whole("av"), "", ind);
+            }
+            if (!first)
+                c += ind + "#pragma unroll\n" + ind + "for (int d = 0; d < " + DBS + "; ++d)\n" + ind + "    #pragma unroll\n" + ind +
+                     "    for (int v = 0; v < 16; ++v) acc[d][v] *= alpha;\n";
+            c += ind + "#pragma unroll\n" + ind + "for (int b = 0; b < " + KBS + "; ++b) sc[b] = sn[b];\n";
+            c += ind + "#pragma unroll\n" + ind + "for (int i = 0; i < " + std::to_string(KT / 16) + "; ++i)\n" + ind +
+                 "    #pragma unroll\n" + ind + "    for (int p = 0; p < 3; ++p) pf[i][p] = pn[i][p];\n";
+            if (!first) c += schedule(ind);
+            c += ind + "__syncthreads();\n";
+            return c;
+        };
+        s += products("sc", "0", "    ") + "    __syncthreads();\n";
+        s += "    {\n        const int it = 0;\n" + iteration(tail != 0 ? partial : "0", true, tail != 0) + "    }\n";
+        if (steps > 1)
+            s += "    for (int it = 1; it < " + std::to_string(steps) + "; ++it) {\n" + iteration(whole("it"), false, false) + "    }\n";
+        s += gather(std::to_string((steps - 1) & 1), "    ");
+
+        // what the split could not hold
+        s += "    sum += __shfl_xor(sum, 32, 64);\n    bool wrong = !(top <= PORCH_FLT_MAX) || !(sum > 0.0f && sum <= PORCH_FLT_MAX), small = false;\n";
+        s += "    #pragma unroll\n    for (int d = 0; d < " + DBS + "; ++d)\n        #pragma unroll\n        for (int v = 0; v < 16; ++v) {\n";
+        s += "            const float x = __builtin_fabsf(acc[d][v]);\n";
+        s += "            wrong |= !(x <= PORCH_FLT_MAX);\n            small |= !(x >= 0x1p-56f);\n        }\n";
+        s += "    const unsigned found = (__ballot(wrong || lowestK < 0x12000000u) != 0 ? 1u : 0u) |\n"
+             "                           (__ballot(small || largest.x >= 0x4e80 || largest.y >= 0x4e80) != 0 ? 2u : 0u) |\n"
+             "                           (__ballot(lowestV < 0x12000000u) != 0 ? 4u : 0u);\n";
+        s += "    if (lane == 0) seen[wave] = found;\n    __syncthreads();\n";
+        s += "    unsigned all = 0;\n    #pragma unroll\n    for (int w = 0; w < " + std::to_string(waves) + "; ++w) all |= seen[w];\n";
+        // In fp32 throughout, in the order of the unfused program: every
+        // row's maximum and sum first, then the weights, divided before they
+        // meet V (undivided, large values could overflow).
+        s += "    if ((all & 1u) != 0 || (all & 6u) == 6u) {\n" + zero_acc;
+        s += "        m = -PORCH_FLT_MAX;\n        sum = 0.0f;\n";
+        s += "        for (int pass = 0; pass < 2; ++pass) {\n        for (int key0 = 0; key0 < " + SK + "; key0 += 32) {\n";
+        s += "            porch_v16f sc;\n            #pragma unroll\n            for (int v = 0; v < 16; ++v) sc[v] = 0.0f;\n";
+        s += "            const idx_t kr = key0 + (lane & 31) < " + SK + " ? key0 + (lane & 31) : " + SK + " - 1;\n";
+        s += "            for (int d = 0; d < " + DD + "; d += 2)\n";
+        s += "                sc = __builtin_amdgcn_mfma_f32_32x32x2f32(K[kr * " + std::to_string(r.k.stride_col) + " + (idx_t)(d + h) * " +
+             std::to_string(r.k.stride_row) + "], Q[q0 * " + std::to_string(r.q.stride_row) + " + (idx_t)(d + h) * " +
+             std::to_string(r.q.stride_col) + "], sc, 0, 0, 0);\n";
+        s += scores("sc", "(idx_t)key0", true, "            ");
+        s += "            if (pass == 0) {\n";
+        s += "                float tm = sc[0];\n                #pragma unroll\n                for (int v = 0; v < 16; ++v) tm = __builtin_fmaxf(tm, sc[v]);\n";
+        s += "                tm = __builtin_fmaxf(tm, __shfl_xor(tm, 32, 64));\n                const float mn = __builtin_fmaxf(m, tm);\n";
+        s += "                float part = 0.0f;\n                #pragma unroll\n                for (int v = 0; v < 16; ++v) part += porch_exp(sc[v] - mn);\n";
+        s += "                sum = sum * porch_exp(m - mn) + part;\n                m = mn;\n            }\n";
+        s += "            else {\n                #pragma unroll\n                for (int v = 0; v < 16; ++v) sc[v] = porch_exp(sc[v] - m) / sum;\n";
+        s += "                #pragma unroll\n                for (int d = 0; d < " + DBS + "; ++d)\n                    #pragma unroll\n                    for (int v = 0; v < 16; ++v) {\n";
+        s += "                        const int key = key0 + 8 * (v >> 2) + 4 * h + (v & 3);\n";
+        s += "                        const float x = key < " + SK + " ? V[(idx_t)key * " + std::to_string(r.v.stride_row) +
+             " + (idx_t)porch_row_dim(d * 32 + (lane & 31)) * " + std::to_string(r.v.stride_col) + "] : 0.0f;\n";
+        s += "                        acc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, sc[v], acc[d], 0, 0, 0);\n";
+        s += "                    }\n            }\n        }\n";
+        s += "        if (pass == 0) sum += __shfl_xor(sum, 32, 64);\n        }\n        sum = 1.0f; // divided already\n    }\n";
+
+        // Output: register v of block d holds dim d 32 + 16 (v / 4 % 2) + 8 h +
+        // 2 (v % 4) + v / 8: eight adjacent dims a lane from four registers of
+        // either half of a block.
+        s += "    if (own < " + SQ + ") {\n";
+        s += "        #pragma unroll\n        for (int d = 0; d < " + DBS + "; ++d)\n        #pragma unroll\n        for (int g = 0; g < 2; ++g) {\n";
+        s += "            float y[8];\n            const idx_t qn = d * 32 + 16 * g + 8 * h;\n";
+        s += "            #pragma unroll\n            for (int e = 0; e < 8; ++e) {\n";
+        s += "                const float acc_v = acc[d][(e & 1) * 8 + 4 * g + (e >> 1)] / sum;\n";
+        s += "                const idx_t q1 = qn + e;\n                (void)q1;\n";
+        {
+            gemm_request e;
+            e.expr = r.expr;
+            e.epilogue = r.epilogue;
+            std::string body;
+            emitter em(*r.expr, body, 1);
+            em.indent = "                ";
+            em.declare_roots({r.epilogue});
+            epilogue_emitter(em, e, r.batched ? std::vector<std::string>{"qb", "q0", "q1"} : std::vector<std::string>{"q0", "q1"},
+                             "acc_v");
+            const std::string v = em.emit(r.epilogue)[0];
+            s += body + "                y[e] = " + v + ";\n            }\n";
+        }
+        s += "            float* const to = out + " + std::string(r.batched ? "(qb * " + SQ + " + q0) * " : "q0 * ") + DD + " + qn;\n";
+        s += "            #pragma unroll\n            for (int e = 0; e < 8; e += 4) {\n";
+        s += "                porch_f4u z = {y[e], y[e + 1], y[e + 2], y[e + 3]};\n                *(porch_f4u*)(to + e) = z;\n            }\n";
+        s += "        }\n    }\n}\n";
+        return kc;
+    }
+
+} // namespace porch::cg

@@ -20,4 +20,8 @@ namespace porch::cg {
     void epilogue_emitter(emitter& em, const gemm_request& r, const std::vector<std::string>& names,
                           const std::string& acc);
 
+    // Device helpers that split fp32 values into three bf16 values
+    // (emit_gemm_split.cpp).
+    const char* bf16_split_helpers();
+
 } // namespace porch::cg

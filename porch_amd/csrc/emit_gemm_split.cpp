@@ -171,7 +171,7 @@ namespace porch::cg {
                 }
                 for (int j = 0; j < 4; ++j) {
                     const std::string J = std::to_string(j);
-                    const std::string p = "(base + o" + id + " + (idx_t)" + std::to_string(j * o.stride_k * 4) + ")";
+                    const std::string p = "(base + o" + id + " + " + std::to_string(j * o.stride_k * 4) + "LL)";
                     const std::string guard = tail == 0 ? "" : "kq" + id + " + " + J + " < " + std::to_string(tail);
                     if (o.how == reading::along_rows) {
                         s += ind + "    porch_f2u v" + id + J + " = {0.0f, 0.0f};\n";
@@ -203,8 +203,10 @@ namespace porch::cg {
             return s;
         }
 
-        const char* helpers() {
-            return R"(typedef float porch_v16f __attribute__((ext_vector_type(16)));
+    } // namespace
+
+    const char* bf16_split_helpers() {
+        return R"(typedef float porch_v16f __attribute__((ext_vector_type(16)));
 typedef float porch_v2f __attribute__((ext_vector_type(2)));
 typedef float porch_f4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float porch_f2u __attribute__((ext_vector_type(2), aligned(4)));
@@ -219,18 +221,22 @@ __device__ __forceinline__ unsigned porch_bf16_pair(float x, float y) {
     const porch_v2f v = {x, y};
     return __builtin_bit_cast(unsigned, __builtin_convertvector(v, porch_b2));
 }
-// Two values as bf16 pairs h + m + l, exactly.  lowest: the least of
-// 2 |bits| - 1 (zeros as the greatest); largest: of the |h|.
+// Two values as bf16 pairs h + m + l, exactly.
+__device__ __forceinline__ void porch_split2(float x, float y, unsigned& h, unsigned& m, unsigned& l) {
+    h = porch_bf16_pair(x, y);
+    const float rx = x - __builtin_bit_cast(float, h << 16), ry = y - __builtin_bit_cast(float, h & 0xffff0000u);
+    m = porch_bf16_pair(rx, ry);
+    l = porch_bf16_pair(rx - __builtin_bit_cast(float, m << 16), ry - __builtin_bit_cast(float, m & 0xffff0000u));
+}
+// The same, noting the least of 2 |bits| - 1 (zeros as the greatest) and the
+// largest |h|.
 __device__ __forceinline__ void porch_split2(float x, float y, unsigned& h, unsigned& m, unsigned& l, unsigned& lowest,
                                              porch_s2& largest) {
     const unsigned ux = (__builtin_bit_cast(unsigned, x) << 1) - 1u, uy = (__builtin_bit_cast(unsigned, y) << 1) - 1u;
     const unsigned u = ux < uy ? ux : uy;
     lowest = u < lowest ? u : lowest;
-    h = porch_bf16_pair(x, y);
+    porch_split2(x, y, h, m, l);
     largest = __builtin_elementwise_max(largest, __builtin_bit_cast(porch_s2, h & 0x7fff7fffu));
-    const float rx = x - __builtin_bit_cast(float, h << 16), ry = y - __builtin_bit_cast(float, h & 0xffff0000u);
-    m = porch_bf16_pair(rx, ry);
-    l = porch_bf16_pair(rx - __builtin_bit_cast(float, m << 16), ry - __builtin_bit_cast(float, m & 0xffff0000u));
 }
 __device__ __forceinline__ void porch_split4(float a, float b, float c, float d, float* to, unsigned& lowest,
                                              porch_s2& largest) {
@@ -244,9 +250,7 @@ __device__ __forceinline__ void porch_split4(float a, float b, float c, float d,
     *(porch_u2*)(to + 8) = l;
 }
 )";
-        }
-
-    } // namespace
+    }
 
     kernel_code emit_gemm_split(const gemm_request& r) {
         const tiling& t = choose(r);
@@ -279,7 +283,7 @@ __device__ __forceinline__ void porch_split4(float a, float b, float c, float d,
         kc.grid_x = static_cast<unsigned>(total * chunks);
         std::string& s = kc.source;
         s = kernel_prologue(r.n_slots, r.width.type());
-        s += helpers();
+        s += bf16_split_helpers();
         s += "extern \"C\" __global__ void __launch_bounds__(512, 2) porch_gemm(" + kernel_params(r.n_slots) + ") {\n";
         // [buffer][slice of 16][octet of k, row][h, m, l: 8 bf16 each].  With
         // the 48-byte pitch 16 consecutive rows meet every bank once per

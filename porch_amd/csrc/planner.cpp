@@ -346,6 +346,148 @@ namespace porch::plan {
             }
 
             // ---------------------------------------------------------
+            // attention: softmax(f(Q K), last axis) V
+            // ---------------------------------------------------------
+            // The nodes of that form under the product `pv`: the scores f and
+            // the product inside f.
+            struct attention_nodes {
+                int f = -1;
+                int qk = -1;
+            };
+            attention_nodes attention_under(int pv) {
+                const attention_nodes none;
+                auto used_by = [&](int x, std::set<int> only) {
+                    const std::vector<int>& u = users[static_cast<size_t>(x)];
+                    return std::set<int>(u.begin(), u.end()) == only;
+                };
+                auto is = [&](int x, ir::op kind) { return x >= 0 && !temp_of.count(x) && g.at(x).kind == kind; };
+                // p = e / bcast(sum(e)), e = exp(f - bcast(max(f))): the
+                // softmax of ops.cpp, each node read only inside it
+                const int p = g.at(pv).lhs;
+                if (!is(p, ir::op::divide) || !used_by(p, {pv})) return none;
+                const int e = g.at(p).lhs, sb = g.at(p).rhs;
+                if (!is(e, ir::op::exp) || !is(sb, ir::op::broadcast) || !used_by(sb, {p})) return none;
+                const int sum = g.at(sb).lhs, d = g.at(e).lhs;
+                if (!is(sum, ir::op::sum) || g.at(sum).lhs != e || !used_by(sum, {sb}) || !used_by(e, {p, sum})) return none;
+                if (!is(d, ir::op::subtract) || !used_by(d, {e})) return none;
+                const int f = g.at(d).lhs, mb = g.at(d).rhs;
+                if (!is(mb, ir::op::broadcast) || !used_by(mb, {d})) return none;
+                const int max = g.at(mb).lhs;
+                if (!is(max, ir::op::max) || g.at(max).lhs != f || !used_by(max, {mb}) || !used_by(f, {d, max})) return none;
+                if (temp_of.count(f)) return none;
+                const std::vector<int64_t>& shape = g.at(f).out;
+                const auto last = static_cast<int64_t>(shape.size()) - 1;
+                if (g.at(p).out != shape || g.at(sb).out != shape || g.at(mb).out != shape) return none;
+                for (const int x : {sum, max})
+                    if (!g.at(x).keepdim || g.at(x).axis != last) return none;
+                // f reads one product, at its own coordinates, and nothing
+                // else reads that product or what f makes of it
+                const int qk = epilogue_matmul(f);
+                if (qk < 0 || g.at(qk).kind != g.at(pv).kind) return none;
+                std::set<int> inside;
+                std::function<bool(int)> closed = [&](int x) {
+                    if (x < 0 || temp_of.count(x) || !depends_on(x, qk) || !inside.insert(x).second) return true;
+                    return x == qk || (closed(g.at(x).lhs) && closed(g.at(x).rhs));
+                };
+                closed(f);
+                for (const int x : inside) {
+                    if (x == f) continue;
+                    for (const int u : users[static_cast<size_t>(x)])
+                        if (!inside.count(u)) return none;
+                }
+                return {f, qk};
+            }
+
+            // An operand of shape [batch, rows, cols] read in place: one
+            // stride over the batch, or one per level where the batch is two
+            // axes merged (the heads of [batch, seq, heads, dim]: a copy of
+            // q, k and v each otherwise).
+            cg::gemm_operand attention_operand(int id, const std::vector<int64_t>& shape) {
+                if (shape.size() == 3 && pure_view_of_input(id)) {
+                    auto affine = [&](int64_t inner) {
+                        cg::kexpr k;
+                        cg::lowering low(g, k, {shape[0] / inner, inner, shape[1], shape[2]});
+                        bind_inputs(low);
+                        cg::ival entry = cg::ival::constant(0, 4);
+                        entry.w = {inner, 1, 0, 0};
+                        const int root = low.at(id, {entry, cg::ival::coordinate(2, 4), cg::ival::coordinate(3, 4)});
+                        const cg::knode& n = k.at(root);
+                        cg::gemm_operand op;
+                        if (n.op != cg::kop::load || !n.index.is_affine) return op;
+                        op.slot = n.slot;
+                        op.offset = n.index.c0;
+                        op.stride_batch_outer = n.index.w[0];
+                        op.stride_batch = n.index.w[1];
+                        op.batch_inner = inner;
+                        op.stride_row = n.index.w[2];
+                        op.stride_col = n.index.w[3];
+                        return op;
+                    };
+                    // (a batch of one level is affine whatever it is cut into)
+                    for (int64_t inner = shape[0]; inner >= 1; --inner) {
+                        if (shape[0] % inner != 0) continue;
+                        const cg::gemm_operand op = affine(inner);
+                        if (op.slot >= 0) return op;
+                    }
+                }
+                return operand(id, shape);
+            }
+
+            bool try_attention(int id, arg_ref dest) {
+                const int pv = epilogue_matmul(id);
+                if (pv < 0) return false;
+                const attention_nodes found = attention_under(pv);
+                if (found.qk < 0) return false;
+                const ir::node& first = g.at(found.qk);
+                const ir::node& second = g.at(pv);
+                const bool batched = second.kind == ir::op::batched_matmul;
+                const size_t o = batched ? 1 : 0;
+                const std::vector<int64_t>& qs = g.at(first.lhs).out;
+                const std::vector<int64_t>& ks = g.at(first.rhs).out;
+                const std::vector<int64_t>& vs = g.at(second.rhs).out;
+                if (!cg::attention_fits(qs[o], ks[o + 1], qs[o + 1], vs[o + 1])) return false;
+                // other reductions and products that f or the epilogue read
+                std::set<int> others;
+                boundaries(found.f, others, {found.qk}, true);
+                for (const int b : others)
+                    if (depends_on(b, found.qk)) return false;
+                std::set<int> after;
+                boundaries(id, after, {pv}, true);
+                for (const int b : after)
+                    if (depends_on(b, pv)) return false;
+                cg::attention_request r;
+                r.batched = batched;
+                r.batch = batched ? qs[0] : 1;
+                r.rows = qs[o];
+                r.keys = ks[o + 1];
+                r.dim = qs[o + 1];
+                r.q = attention_operand(first.lhs, qs);
+                r.k = attention_operand(first.rhs, ks);
+                r.v = attention_operand(second.rhs, vs);
+                for (const int b : others) ensure_temp(b);
+                for (const int b : after) ensure_temp(b);
+                auto lowered = [&](cg::kexpr& k, int root, int product) {
+                    cg::lowering low(g, k, g.at(product).out);
+                    bind_inputs(low);
+                    cg::binding acc;
+                    acc.what = cg::binding::kind::row_value;
+                    acc.row = 0;
+                    low.bound[product] = acc;
+                    return low.at(root, low.identity());
+                };
+                cg::kexpr ks_expr, kv_expr;
+                r.score = lowered(ks_expr, found.f, found.qk);
+                r.score_expr = &ks_expr;
+                r.epilogue = lowered(kv_expr, id, pv);
+                r.expr = &kv_expr;
+                r.n_slots = n_slots();
+                r.width = width;
+                r.compute_units = compute_units;
+                add_step(cg::emit_attention(r), dest);
+                return true;
+            }
+
+            // ---------------------------------------------------------
             // row programs
             // ---------------------------------------------------------
             // Collects the row reductions under `id` (through elementwise
@@ -714,6 +856,7 @@ namespace porch::plan {
                     emit_identity_fill(id, dest);
                     return;
                 }
+                if (try_attention(id, dest)) return;
                 if (try_gemm(id, dest)) return;
                 if (try_row(id, dest)) return;
                 if (ir::is_reduction(n.kind)) {

@@ -1,0 +1,200 @@
+"""softmax(f(q k^T)) v in one kernel: tile remainders, operand layouts,
+masks, head dimensions, the plans that take it and those that don't, and the
+values its bf16 split cannot hold."""
+
+import numpy as np
+import pytest
+
+import porch_amd as porch
+from tests.helpers import placeholder
+from tests.kernel_emu import emulate as emu
+
+
+def attention(q, k, v, scale, mask=None):
+    """q [b, sq, d], k [b, sk, d], v [b, sk, d]."""
+    scores = porch.batched_matmul(q, porch.permute(k, [0, 2, 1])) * scale
+    if mask is not None:
+        scores = scores + porch.broadcast_to(mask, scores.shape())
+    return porch.batched_matmul(porch.softmax(scores, 2), v)
+
+
+def reference(q, k, v, scale, mask=None):
+    s = np.matmul(q.astype(np.float64), k.astype(np.float64).transpose(0, 2, 1)) * np.float64(np.float32(scale))
+    if mask is not None:
+        s = s + mask
+    with np.errstate(invalid="ignore", over="ignore"):
+        top = np.maximum(np.max(np.where(np.isnan(s), -np.inf, s), -1, keepdims=True), -np.finfo(np.float32).max)
+        p = np.exp(s - top)
+        p = p / p.sum(-1, keepdims=True)
+        return np.matmul(p, v.astype(np.float64)), np.matmul(p, np.abs(v.astype(np.float64)))
+
+
+def close(got, want, scale):
+    """Sums of `dim` products inside exp, then of weights: each rounding of a
+    score moves its weight by as much, relatively; 64 covers dim and the
+    scores' size here (|s| up to about 8)."""
+    with np.errstate(over="ignore"):
+        want32 = want.astype(np.float32)
+    assert np.array_equal(np.isnan(got), np.isnan(want32))
+    assert np.array_equal(got[np.isinf(want32)], want32[np.isinf(want32)])
+    ok = np.isfinite(want32)
+    assert np.all(np.abs(got[ok] - want[ok]) <= 64 * 2.0 ** -23 * scale[ok] + 1e-37)
+
+
+# (batch, queries, keys, dim, masked): around the tiles of 32 queries, of
+# 128 / 64 / 32 keys (dim 32 / 64 / 128), keys of one partial tile alone,
+# none, and one past; 40 entries take workgroups of eight waves
+SIZES = [(1, 32, 32, 64, False), (2, 33, 64, 64, True), (1, 127, 65, 64, False), (3, 129, 200, 64, True),
+         (1, 40, 130, 32, True), (2, 100, 128, 32, False), (1, 64, 33, 128, True), (2, 70, 96, 128, False),
+         (40, 1000, 321, 64, False), (40, 900, 100, 128, True), (40, 900, 300, 32, False)]
+
+
+def inputs(size, rng):
+    b, sq, sk, d, masked = size
+    q, k, v = (rng.standard_normal((b, n, d)).astype(np.float32) for n in (sq, sk, sk))
+    mask = np.where(rng.random((1, sq, sk)) < 0.3, np.float32(-1e9), np.float32(0)) if masked else None
+    return q, k, v, mask
+
+
+def graph(make, q, k, v, mask):
+    return attention(make(q), make(k), make(v), q.shape[2] ** -0.5, None if mask is None else make(mask))
+
+
+def host_only(x):
+    return placeholder(list(x.shape), np.ascontiguousarray(x, np.float32).reshape(-1))
+
+
+def emulated(q, k, v, mask):
+    expr = graph(host_only, q, k, v, mask)
+    assert [x["kind"] for x in porch.plan(expr)["kernels"]] == ["attention"]
+    assert all(r["ok"] for r in emu.emulate(expr, timeout=300))
+    values = [q, k] + ([] if mask is None else [mask]) + [v]
+    return emu.evaluate(expr, values, timeout=300)
+
+
+@pytest.mark.skipif(not emu.available(), reason="no clang for the emulation")
+@pytest.mark.parametrize("size", [(1, 33, 70, 64, True), (1, 32, 33, 128, False)])
+def test_emulated(size):
+    q, k, v, mask = inputs(size, np.random.default_rng(1))
+    want, scale = reference(q, k, v, size[3] ** -0.5, mask)
+    close(emulated(q, k, v, mask), want, scale)
+
+
+def special(name, q, k, v, mask):
+    if name == "infinite value":
+        v[0, 5, 3] = np.inf
+    elif name == "nan key":
+        k[0, 7, 1] = np.nan
+    elif name == "large values":
+        v *= np.float32(1e38)
+    elif name == "tiny queries and keys":
+        q *= np.float32(1e-36)
+        k[:] = np.where(np.abs(k) < 1.5, np.float32(0.0), k) * np.float32(1e36)
+    elif name == "tiny values":
+        v *= np.float32(1e-37)
+    elif name == "masked rows":
+        mask[0, :3] = -np.inf
+    elif name == "masked to the lowest value":
+        mask[0, 1] = -np.finfo(np.float32).max
+        mask[0, 2, 4:] = -np.inf
+
+
+SPECIAL = ["infinite value", "nan key", "large values", "tiny queries and keys", "tiny values", "masked rows",
+           "masked to the lowest value"]
+
+
+@pytest.mark.skipif(not emu.available(), reason="no clang for the emulation")
+@pytest.mark.parametrize("name", ["infinite value", "masked rows", "tiny values"])
+def test_emulated_special_values(name):
+    size = (1, 34, 70, 64, True)
+    q, k, v, mask = inputs(size, np.random.default_rng(2))
+    special(name, q, k, v, mask)
+    with np.errstate(invalid="ignore"):
+        want, scale = reference(q, k, v, 0.125, mask)
+    close(emulated(q, k, v, mask), want, scale)
+
+
+def kinds(expr):
+    return [x["kind"] for x in porch.plan(expr)["kernels"]]
+
+
+def test_plans():
+    P = placeholder
+    d = 64
+    q, k, v = P([4, 128, d]), P([4, 256, d]), P([4, 256, d])
+    assert kinds(attention(q, k, v, 0.125)) == ["attention"]
+    assert kinds(porch.relu(attention(q, k, v, 0.125)) + 1.0) == ["attention"]
+    # rank 2, k stored transposed
+    s = porch.matmul(P([64, 32]), P([32, 96])) * 0.5
+    assert kinds(porch.matmul(porch.softmax(s, 1), P([96, 32]))) == ["attention"]
+    # other head dimensions, fewer than 32 rows, another axis
+    for shape in ([4, 128, 48], [4, 128, 256], [4, 20, 64]):
+        assert "attention" not in kinds(attention(P(shape), P(shape), P(shape), 0.125))
+    s = porch.batched_matmul(q, porch.permute(k, [0, 2, 1]))
+    assert "attention" not in kinds(porch.batched_matmul(porch.softmax(s, 1), v))
+    # the weights or the scores are read elsewhere too
+    p = porch.softmax(s, 2)
+    both = porch.batched_matmul(p, v) + porch.broadcast_to(porch.sum(p, 2, True), [4, 128, d])
+    assert "attention" not in kinds(both)
+    both = porch.batched_matmul(p, v) + porch.broadcast_to(porch.max(s * 2.0, 2, True), [4, 128, d])
+    assert "attention" not in kinds(both)
+    # a softmax in all but its last step
+    e = porch.exp(s - porch.broadcast_to(porch.max(s, 2, True), s.shape()))
+    assert "attention" not in kinds(porch.batched_matmul(e, v))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("size", SIZES)
+def test_sizes(gpu, size):
+    q, k, v, mask = inputs(size, np.random.default_rng(3))
+    expr = graph(lambda x: gpu.tensor(list(x.shape), x.reshape(-1)), q, k, v, mask)
+    assert kinds(expr) == ["attention"]
+    want, scale = reference(q, k, v, size[3] ** -0.5, mask)
+    close(gpu.materialize(expr).cpu().reshape(want.shape), want, scale)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", SPECIAL)
+def test_special_values(gpu, name):
+    for size in [(1, 34, 70, 64, True), (2, 200, 130, 32, True)]:
+        q, k, v, mask = inputs(size, np.random.default_rng(4))
+        special(name, q, k, v, mask)
+        with np.errstate(invalid="ignore"):
+            want, scale = reference(q, k, v, size[3] ** -0.5, mask)
+        expr = graph(lambda x: gpu.tensor(list(x.shape), x.reshape(-1)), q, k, v, mask)
+        assert kinds(expr) == ["attention"]
+        got = gpu.materialize(expr).cpu().reshape(want.shape)
+        close(got, want, scale)
+
+
+def layouts(make, rng):
+    """Every way a tile is read: q, k, v interleaved by heads (one read in
+    place), k^T and v^T stored, and strided along both."""
+    b, s, d = 2, 75, 64
+    x = [rng.standard_normal((b, s, d)).astype(np.float32) for _ in range(3)]
+    heads = [np.ascontiguousarray(a.transpose(1, 0, 2)) for a in x]
+    yield x, [porch.permute(make(a), [1, 0, 2]) for a in heads]
+    turned = [np.ascontiguousarray(a.transpose(0, 2, 1)) for a in x]
+    yield x, [porch.permute(make(a), [0, 2, 1]) for a in turned]
+    # two entries of three heads each, in [batch, seq, heads, dim]
+    six = [rng.standard_normal((6, s, d)).astype(np.float32) for _ in range(3)]
+    apart = [np.ascontiguousarray(a.reshape(2, 3, s, d).transpose(0, 2, 1, 3)) for a in six]
+    yield six, [porch.reshape(porch.permute(make(a), [0, 2, 1, 3]), [6, s, d]) for a in apart]
+    wide = []
+    for a in x:
+        w = np.zeros((b, 2 * s, 2 * d), np.float32)
+        w[:, 1::2, ::2] = a
+        wide.append(w)
+    yield x, [make(w)[porch.all, porch.slice(1, 2 * s, 2), porch.slice(0, 2 * d, 2)] for w in wide]
+
+
+def test_layouts_are_read_in_place():
+    for _, views in layouts(host_only, np.random.default_rng(5)):
+        assert kinds(attention(*views, 0.125)) == ["attention"]
+
+
+@pytest.mark.gpu
+def test_layouts(gpu):
+    for x, views in layouts(lambda a: gpu.tensor(list(a.shape), a.reshape(-1)), np.random.default_rng(5)):
+        want, scale = reference(*x, 0.125)
+        close(gpu.materialize(attention(*views, 0.125)).cpu().reshape(want.shape), want, scale)
