@@ -556,21 +556,42 @@ namespace porch::cg {
 
     int64_t gemm_k_chunks(const gemm_request& r) {
         if (!uses_mfma(r)) return 1;
-        // 128 x 128 tiles (the smaller of the split kernel's); split K when they leave over half the compute units idle
-        // and K is long (1024 or more: a shorter loop finishes within the
-        // time of the extra combine launch), into the fewest chunks
-        // (dividing the K-steps, each at least 8 of them) that give two
-        // workgroups per compute unit.
+        // Split K where 128 x 128 tiles leave over half the compute units
+        // idle and K is over 512 (a shorter loop takes at most 16 steps of
+        // 32, of which a second launch leaves little to save).  From K of
+        // 1024 on, into the fewest equal chunks of 16-wide steps, each at
+        // least 8 of them, that give two workgroups per compute unit; where
+        // the steps have no such divisor, or the estimate below says that
+        // uneven chunks take half the time, by the estimate.
+        // Unsplit or equal chunks / by the estimate: 400 x 776 x 724 35.4 /
+        // 14.5 us, 28 x 3393 x 1770 47.2 / 16.3, 2149 x 896 x 455 40.2 /
+        // 21.9; the gradients of a 2666 x 212 x 3712 layer 179 / 87.
         const int64_t cus = std::max(r.compute_units, 8);
         const int64_t tiles = ((r.m + BM - 1) / BM) * ((r.n + BN - 1) / BN) * r.batch;
-        const int64_t steps = (r.k + BK - 1) / BK;
-        if (2 * tiles >= cus || steps < 64) return 1;
+        if (2 * tiles >= cus || r.k <= 512) return 1;
+        const int64_t narrow_steps = (r.k + BK - 1) / BK;
         int64_t best = 1;
-        for (int64_t d = 2; d * 8 <= steps; ++d) {
-            if (steps % d != 0) continue;
-            best = d;
-            if (tiles * d >= 2 * cus) break;
-        }
+        if (narrow_steps >= 64)
+            for (int64_t d = 2; d * 8 <= narrow_steps; ++d) {
+                if (narrow_steps % d != 0) continue;
+                best = d;
+                if (tiles * d >= 2 * cus) break;
+            }
+        // In steps over 32 values of K (1.4 us each): rounds of workgroups
+        // over the compute units times the steps of each, and for a split the
+        // combine's launch and the partial sums' way through memory, 8 bytes
+        // an output and chunk at 4 TB/s.
+        const int64_t steps = (r.k + 31) / 32, outputs = r.batch * r.m * r.n;
+        auto cost = [&](int64_t d) {
+            const double loop = static_cast<double>(((tiles * d + cus - 1) / cus) * ((steps + d - 1) / d));
+            return d == 1 ? loop : loop + 2.8 + static_cast<double>(d * outputs * 8) / 5.6e6;
+        };
+        double least = cost(best) * (best == 1 ? 0.9 : 0.5);
+        for (int64_t d = 2; d <= std::min<int64_t>(steps / 2, 64) && d * outputs < (int64_t{1} << 28); ++d)
+            if (cost(d) < least) {
+                least = cost(d);
+                best = d;
+            }
         return best;
     }
 

@@ -38,6 +38,9 @@ SMALL = {
     "split K, partial step": ([40, 1030], [1030, 37], lambda a, b: porch.matmul(a, b) + 1.0),
 }
 
+# chunks of K with uneven numbers of steps: 17 whole ones (the fewest that are split), 16 and a partial one
+UNEVEN = {"whole steps": (70, 544, 131), "partial step": (129, 515, 40), "odd K, odd columns": (33, 1001, 257)}
+
 
 def build(name, make):
     sa, sb, f = SMALL[name]
@@ -61,6 +64,31 @@ def test_emulated_products_bit_exact(name):
     assert all(r["ok"] for r in emu.emulate(expr, timeout=300))
     got = emu.evaluate(expr, [a, b], timeout=300)
     assert np.array_equal(got, host.evaluate(expr).reshape(got.shape))
+
+
+def uneven(name, make, rng):
+    m, k, n = UNEVEN[name]
+    a, b, c = ints((m, k), rng), ints((k, n), rng), ints((1, n), rng)
+    expr = porch.relu(porch.matmul(make(a), make(b)) + porch.broadcast_to(make(c), [m, n])) - 0.5
+    assert [x["kind"] for x in porch.plan(expr)["kernels"]] == ["gemm.mfma", "gemm.combine"]
+    return [a, b, c], expr
+
+
+@pytest.mark.skipif(not emu.available(), reason="no clang for the emulation")
+@pytest.mark.parametrize("name", sorted(UNEVEN))
+def test_emulated_uneven_chunks(name):
+    values, expr = uneven(name, lambda x: filled(list(x.shape), x), np.random.default_rng(7))
+    assert all(r["ok"] for r in emu.emulate(expr, timeout=300))
+    got = emu.evaluate(expr, values, timeout=300)
+    assert np.array_equal(got, host.evaluate(expr).reshape(got.shape))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", sorted(UNEVEN))
+def test_uneven_chunks(gpu, name):
+    _, expr = uneven(name, lambda x: gpu.tensor(list(x.shape), x.reshape(-1)), np.random.default_rng(8))
+    out = gpu.materialize(expr).cpu().reshape(expr.shape())
+    assert np.array_equal(out, host.evaluate(expr).reshape(out.shape))
 
 
 @pytest.mark.skipif(not emu.available(), reason="no clang for the emulation")
