@@ -18,6 +18,9 @@
 // registers; a row's maximum and sum need one exchange between the lane's
 // two halves of the wave.
 //
+// Few queries leave most of the chip idle that way: there the waves of a
+// workgroup split the keys of one block of 32 queries (see key_split).
+//
 // An iteration computes the products of the next tile, the weights of this
 // one and the sums of the one before: independent of each other, so that a
 // wave's MFMAs run beside its exps and splits (up to six vector instructions
@@ -192,6 +195,22 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
 )";
         }
 
+        // Waves among which the keys of a block of 32 queries are split; 0:
+        // none.  A workgroup of shared tiles walks all keys for 128 queries
+        // or more, which leaves compute units idle where there are few; with
+        // split keys each wave splits its own K and V into bf16 values, twice
+        // the vector work.  Shared / split, causal: dim 64, 8 heads of 128
+        // positions 14.8 / 9.9 us, 4 of 1000 (128 blocks) 89 / 32, 8 of 2048
+        // (512) 139 / 104; dim 32, 16 of 1000 (512) 76 / 32; dim 128, 4 of
+        // 2048 (256) 226 / 106, 24 of 512 (384) 70 / 71, 16 of 1000 (512) 116
+        // / 135: up to two rounds of blocks, one at dim 128, where four waves
+        // fill a compute unit's registers.
+        int key_split(const attention_request& r) {
+            const int64_t blocks = r.batch * ((r.rows + 31) / 32);
+            if (blocks > (r.dim == 128 ? 1 : 2) * static_cast<int64_t>(std::max(r.compute_units, 8))) return 0;
+            return r.dim == 128 || r.keys <= 128 ? 4 : 8;
+        }
+
     } // namespace
 
     bool attention_fits(int64_t rows, int64_t keys, int64_t dim, int64_t value_dim) {
@@ -202,14 +221,16 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
         if (!attention_fits(r.rows, r.keys, r.dim, r.dim)) throw std::logic_error("emit_attention: shape");
         const int D = static_cast<int>(r.dim);
         // keys a tile: two buffers of K and V in 48 KB of LDS (96 at dim 128)
-        const int KT = std::max(32, 2048 / D);
+        const int KT = key_split(r) > 0 ? 32 : std::max(32, 2048 / D);
         const int KB = KT / 32, DB = D / 32, DS = D / 16;
+        const bool apart = D == 32; // see gather
         // Eight waves (256 queries) a workgroup share each tile of K and V;
         // four where that still leaves no compute unit a second workgroup.
         const int64_t cus = std::max(r.compute_units, 8);
-        const int waves = r.batch * ((r.rows + 127) / 128) <= cus ? 4 : 8;
+        const int split = key_split(r);
+        const int waves = split > 0 ? split : r.batch * ((r.rows + 127) / 128) <= cus ? 4 : 8;
         const int threads = 64 * waves;
-        const int BQ = 32 * waves;
+        const int BQ = split > 0 ? 32 : 32 * waves;
         const int64_t tiles = (r.rows + BQ - 1) / BQ;
         const int64_t total = tiles * r.batch;
         const int64_t full = r.keys / KT, tail = r.keys % KT;
@@ -232,9 +253,15 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
         s += helpers();
         s += "extern \"C\" __global__ void __launch_bounds__(" + std::to_string(threads) + ", " + (waves == 8 ? "2" : "1") +
              ") porch_attention(" + kernel_params(r.n_slots) + ") {\n";
-        s += "    __shared__ __attribute__((aligned(16))) float Ks[2][" + DSS + "][" + std::to_string(2 * KT) + "][12];\n";
-        s += "    __shared__ __attribute__((aligned(16))) float Vs[2][" + std::to_string(KT / 16) + "][" +
-             std::to_string(2 * D) + "][12];\n";
+        if (split > 0) {
+            s += "    __shared__ float parts[" + std::to_string(waves) + "][" + std::to_string(16 * DB) + "][64];\n";
+            s += "    __shared__ float maxima[" + std::to_string(waves) + "][32], sums[" + std::to_string(waves) + "][32];\n";
+        }
+        else {
+            s += "    __shared__ __attribute__((aligned(16))) float Ks[2][" + DSS + "][" + std::to_string(2 * KT) + "][12];\n";
+            s += "    __shared__ __attribute__((aligned(16))) float Vs[2][" + std::to_string(KT / 16) + "][" +
+                 std::to_string(2 * D) + "][12];\n";
+        }
         s += "    __shared__ unsigned seen[8];\n";
         s += "    const int tid = threadIdx.x;\n    const int lane = tid & 63;\n    const int wave = tid >> 6;\n";
         s += "    const int h = lane >> 5;\n";
@@ -246,7 +273,7 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
              " + blockIdx.x / 8;\n";
         if (r.batched) s += "    const idx_t qb = lin / " + std::to_string(tiles) + ";\n";
         s += "    const idx_t own = (lin" + (r.batched ? " % " + std::to_string(tiles) : std::string()) + ") * " +
-             std::to_string(BQ) + " + wave * 32 + (lane & 31);\n";
+             std::to_string(BQ) + (split > 0 ? "" : " + wave * 32") + " + (lane & 31);\n";
         s += "    const idx_t q0 = own < " + SQ + " ? own : (idx_t)" + SQ + " - 1;\n";
         auto base = [&](const char* x, const gemm_operand& op) {
             s += std::string("    const float* __restrict__ ") + x + " = a" + std::to_string(op.slot) + " + " +
@@ -261,14 +288,15 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
         base("Q", r.q);
         base("K", r.k);
         base("V", r.v);
-        s += setup_code(K, threads, OT) + setup_code(V, threads, OT);
+        if (split == 0) s += setup_code(K, threads, OT) + setup_code(V, threads, OT);
         s += "    unsigned lowestK = 0xffffffffu, lowestV = 0xffffffffu;\n    porch_s2 largest = {0, 0};\n";
         const std::string partial = std::to_string(full * KT);
         const std::string ahead_of = tail != 0 ? " - 1" : "";
         auto whole = [&](const std::string& g) { return "(" + g + ahead_of + ") * " + KTS; };
         // the partial tile first, so that the loop's loads need no tests
         const std::string valid = tail != 0 ? std::to_string(tail) : "";
-        s += load_code(K, tail != 0 ? partial : "0", valid, "    ") + load_code(V, tail != 0 ? partial : "0", valid, "    ");
+        if (split == 0)
+            s += load_code(K, tail != 0 ? partial : "0", valid, "    ") + load_code(V, tail != 0 ? partial : "0", valid, "    ");
         // this lane's query, split
         s += "    porch_b8 qf[" + DSS + "][3];\n";
         s += "    #pragma unroll\n    for (int t = 0; t < " + DSS + "; ++t) {\n        porch_u4 u[3];\n";
@@ -278,15 +306,16 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
         s += "            porch_split2(Q[at], Q[at + " + std::to_string(r.q.stride_col) + "], x, y, z, lowestK, largest);\n";
         s += "            u[0][e] = x; u[1][e] = y; u[2][e] = z;\n        }\n";
         s += "        #pragma unroll\n        for (int p = 0; p < 3; ++p) qf[t][p] = __builtin_bit_cast(porch_b8, u[p]);\n    }\n";
-        s += store_code(K, "0", "    ");
-        if (steps > 1) {
+        if (split == 0) s += store_code(K, "0", "    ");
+        if (split == 0 && steps > 1) {
             s += load_code(K, whole("1"), "", "    ") + store_code(K, "1", "    ");
             s += load_code(K, whole(steps > 2 ? "2" : "1"), "", "    ");
         }
-        s += "    float m = -0x1p100f, sum = 0.0f, top = 0.0f;\n    porch_v16f acc[" + DBS + "], sc[" + KBS + "];\n    porch_b8 pf[" + std::to_string(KT / 16) + "][3];\n";
+        s += "    float m = -0x1p100f, sum = 0.0f, top = 0.0f, al = 1.0f;\n    (void)al;\n    porch_v16f acc[" + DBS + "], sc[" + KBS + "];\n    porch_b8 pf[" + std::to_string(KT / 16) + "][3];\n";
         const std::string zero_acc = "    #pragma unroll\n    for (int d = 0; d < " + DBS +
                                      "; ++d)\n        #pragma unroll\n        for (int v = 0; v < 16; ++v) acc[d][v] = 0.0f;\n";
-        s += zero_acc + "    __syncthreads();\n";
+        s += zero_acc;
+        if (split == 0) s += "    __syncthreads();\n";
 
         // f of the 16 products sc[kb][..] of keys key0 + kb 32 + 8 g + 4 h + j
         const bool vec = vector_scores(*r.score_expr, r.score);
@@ -409,9 +438,20 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
                  "[t][p] = __builtin_bit_cast(porch_b8, u[p]);\n" + ind + "}\n";
             return c;
         };
-        // acc += V^T P^T for the weights in pf and V's buffer `vb`
+        // V^T P^T for the weights in pf and V's buffer `vb`, onto the output.
+        // At dim 32 a tile's product is summed by itself, in two chains of
+        // MFMAs, and added to the output scaled by `al`, the factor of the
+        // maximum before: an output has one rounding a tile at its own size,
+        // not one per MFMA (24 heads of 2432 positions: error against 64
+        // bits 3.1e-7, and 8.0e-7 with the MFMAs on the output, where the
+        // unfused program has 5.1e-7; 126 us against 122).
         auto gather = [&](const std::string& vb, const std::string& ind) {
             std::string c;
+            const std::string sums = apart ? "tile[t & 1][d]" : "acc[d]";
+            if (apart)
+                c += ind + "porch_v16f tile[2][" + DBS + "];\n" + ind + "#pragma unroll\n" + ind + "for (int d = 0; d < " + DBS +
+                     "; ++d)\n" + ind + "    #pragma unroll\n" + ind +
+                     "    for (int v = 0; v < 16; ++v) tile[0][d][v] = tile[1][d][v] = 0.0f;\n";
             c += ind + "#pragma unroll\n" + ind + "for (int t = 0; t < " + std::to_string(KT / 16) + "; ++t) {\n";
             c += ind + "    const int row = (lane & 31) ^ ((2 * t + h) * " + std::to_string(swizzle_of(V)) + ");\n";
             c += ind + "    porch_b8 vf[" + DBS + "][3];\n";
@@ -419,10 +459,14 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
                  ind + "        for (int p = 0; p < 3; ++p) vf[d][p] = *(const porch_b8*)&Vs[" + vb + "][t][h * " + DD +
                  " + d * 32 + row][p * 4];\n";
             for (const auto& pr : pairs)
-                c += ind + "    #pragma unroll\n" + ind + "    for (int d = 0; d < " + DBS +
-                     "; ++d) acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[d][" + std::to_string(pr[0]) + "], pf[t][" +
-                     std::to_string(pr[1]) + "], acc[d], 0, 0, 0);\n";
-            return c + ind + "}\n";
+                c += ind + "    #pragma unroll\n" + ind + "    for (int d = 0; d < " + DBS + "; ++d) " + sums +
+                     " = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[d][" + std::to_string(pr[0]) + "], pf[t][" +
+                     std::to_string(pr[1]) + "], " + sums + ", 0, 0, 0);\n";
+            c += ind + "}\n";
+            if (apart)
+                c += ind + "#pragma unroll\n" + ind + "for (int d = 0; d < " + DBS + "; ++d)\n" + ind + "    #pragma unroll\n" + ind +
+                     "    for (int v = 0; v < 16; ++v) acc[d][v] = __builtin_fmaf(acc[d][v], al, tile[0][d][v] + tile[1][d][v]);\n";
+            return c;
         };
         // Iteration `it`: the products of tile it + 1, the weights of tile it
         // and the sums of tile it - 1 are independent, so that one wave's MFMAs
@@ -443,7 +487,8 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
                 c += ind + "const int av = it + 1 < " + std::to_string(steps) + " ? it + 1 : " + std::to_string(steps - 1) + ";\n";
                 c += load_code(V, whole("av"), "", ind);
             }
-            if (!first)
+            if (apart) c += ind + "al = alpha;\n";
+            else if (!first)
                 c += ind + "#pragma unroll\n" + ind + "for (int d = 0; d < " + DBS + "; ++d)\n" + ind + "    #pragma unroll\n" + ind +
                      "    for (int v = 0; v < 16; ++v) acc[d][v] *= alpha;\n";
             c += ind + "#pragma unroll\n" + ind + "for (int b = 0; b < " + KBS + "; ++b) sc[b] = sn[b];\n";
@@ -453,14 +498,102 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
             c += ind + "__syncthreads();\n";
             return c;
         };
-        s += products("sc", "0", "    ") + "    __syncthreads();\n";
-        s += "    {\n        const int it = 0;\n" + iteration(tail != 0 ? partial : "0", true, tail != 0) + "    }\n";
-        if (steps > 1)
-            s += "    for (int it = 1; it < " + std::to_string(steps) + "; ++it) {\n" + iteration(whole("it"), false, false) + "    }\n";
-        s += gather(std::to_string((steps - 1) & 1), "    ");
+        // Split keys: wave w takes the tiles w, w + waves, .. and reads their
+        // fragments from memory as the MFMAs want them (lane: a key of K, a
+        // dim of V, eight values along the product); no wave waits for
+        // another until the end.
+        auto fragments = [&](const std::string& key0, bool masked, const std::string& ind) {
+            std::string c;
+            const std::string limit = " < " + SK + " ? kx : (idx_t)" + SK + " - 1";
+            c += ind + "#pragma unroll\n" + ind + "for (int t = 0; t < " + DSS + "; ++t)\n" + ind + "    #pragma unroll\n" + ind +
+                 "    for (int b = 0; b < " + KBS + "; ++b) {\n";
+            c += ind + "        const idx_t kx = " + key0 + " + b * 32 + (lane & 31);\n";
+            c += ind + "        const float* const at = K + (" + (masked ? "kx" + limit : std::string("kx")) + ") * " +
+                 std::to_string(r.k.stride_col) + " + (idx_t)(t * 16 + h * 8) * " + std::to_string(r.k.stride_row) + ";\n";
+            if (r.k.stride_row == 1)
+                c += ind + "        const porch_f4u x = *(const porch_f4u*)at, y = *(const porch_f4u*)(at + 4);\n" + ind +
+                     "        #pragma unroll\n" + ind + "        for (int e = 0; e < 4; ++e) { kr[t][b][e] = x[e]; kr[t][b][4 + e] = y[e]; }\n";
+            else
+                c += ind + "        #pragma unroll\n" + ind + "        for (int e = 0; e < 8; ++e) kr[t][b][e] = at[(idx_t)e * " +
+                     std::to_string(r.k.stride_row) + "];\n";
+            c += ind + "    }\n";
+            c += ind + "#pragma unroll\n" + ind + "for (int t = 0; t < " + std::to_string(KT / 16) + "; ++t)\n" + ind +
+                 "    #pragma unroll\n" + ind + "    for (int d = 0; d < " + DBS + "; ++d) {\n";
+            c += ind + "        const float* const at = V + (idx_t)(d * 32 + porch_row_dim(lane & 31)) * " +
+                 std::to_string(r.v.stride_col) + ";\n";
+            if (r.v.stride_row == 1 && !masked)
+                c += ind + "        const porch_f4u x = *(const porch_f4u*)(at + " + key0 + " + t * 16 + 4 * h), y = *(const porch_f4u*)(at + " +
+                     key0 + " + t * 16 + 4 * h + 8);\n" + ind +
+                     "        #pragma unroll\n" + ind + "        for (int e = 0; e < 4; ++e) { vr[t][d][e] = x[e]; vr[t][d][4 + e] = y[e]; }\n";
+            else
+                c += ind + "        #pragma unroll\n" + ind + "        for (int e = 0; e < 8; ++e) {\n" + ind +
+                     "            const idx_t kx = " + key0 + " + t * 16 + 4 * h + (e & 3) + (e & 4) * 2;\n" + ind +
+                     "            vr[t][d][e] = at[(" + (masked ? "kx" + limit : std::string("kx")) + ") * " + std::to_string(r.v.stride_row) +
+                     "];\n" + ind + "        }\n";
+            return c + ind + "    }\n";
+        };
+        auto own_tile = [&](bool masked) {
+            const std::string ind = "            ";
+            std::string c = fragments("key0", masked, ind);
+            auto split8 = [&](const std::string& from, const std::string& lowest) {
+                return ind + "    porch_b8 f[3];\n" + ind + "    {\n" + ind + "        porch_u4 u[3];\n" + ind +
+                       "        #pragma unroll\n" + ind + "        for (int e = 0; e < 4; ++e) {\n" + ind +
+                       "            unsigned x, y, z;\n" + ind + "            porch_split2(" + from + "[2 * e], " + from +
+                       "[2 * e + 1], x, y, z, " + lowest + ", largest);\n" + ind +
+                       "            u[0][e] = x; u[1][e] = y; u[2][e] = z;\n" + ind + "        }\n" + ind +
+                       "        #pragma unroll\n" + ind + "        for (int p = 0; p < 3; ++p) f[p] = __builtin_bit_cast(porch_b8, u[p]);\n" +
+                       ind + "    }\n";
+            };
+            c += ind + "#pragma unroll\n" + ind + "for (int b = 0; b < " + KBS + "; ++b)\n" + ind +
+                 "    #pragma unroll\n" + ind + "    for (int v = 0; v < 16; ++v) sc[b][v] = 0.0f;\n";
+            c += ind + "#pragma unroll\n" + ind + "for (int b = 0; b < " + KBS + "; ++b)\n" + ind + "#pragma unroll\n" + ind +
+                 "for (int t = 0; t < " + DSS + "; ++t) {\n" + split8("kr[t][b]", "lowestK");
+            for (const auto& pr : pairs)
+                c += ind + "    sc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[" + std::to_string(pr[0]) + "], qf[t][" +
+                     std::to_string(pr[1]) + "], sc[b], 0, 0, 0);\n";
+            c += ind + "}\n";
+            c += weights("key0", masked, "pf", ind);
+            c += ind + "#pragma unroll\n" + ind + "for (int d = 0; d < " + DBS + "; ++d) {\n";
+            c += ind + "    porch_v16f own_sum;\n" + ind + "    #pragma unroll\n" + ind + "    for (int v = 0; v < 16; ++v) own_sum[v] = 0.0f;\n";
+            c += ind + "    #pragma unroll\n" + ind + "    for (int t = 0; t < " + std::to_string(KT / 16) + "; ++t) {\n" + split8("vr[t][d]", "lowestV");
+            for (const auto& pr : pairs)
+                c += ind + "        own_sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[" + std::to_string(pr[0]) + "], pf[t][" +
+                     std::to_string(pr[1]) + "], own_sum, 0, 0, 0);\n";
+            c += ind + "    }\n";
+            c += ind + "    #pragma unroll\n" + ind + "    for (int v = 0; v < 16; ++v) acc[d][v] = __builtin_fmaf(acc[d][v], alpha, own_sum[v]);\n" + ind + "}\n";
+            return c;
+        };
+        if (split > 0) {
+            s += "    float kr[" + DSS + "][" + KBS + "][8], vr[" + std::to_string(KT / 16) + "][" + DBS + "][8];\n";
+            s += "    for (int it = wave; it < " + std::to_string(steps) + "; it += " + std::to_string(waves) + ") {\n";
+            s += "        const idx_t key0 = (idx_t)it * " + KTS + ";\n";
+            if (tail == 0) s += "        {\n" + own_tile(false) + "        }\n    }\n";
+            else if (full == 0) s += "        {\n" + own_tile(true) + "        }\n    }\n";
+            else
+                s += "        if (it < " + std::to_string(full) + ") {\n" + own_tile(false) + "        }\n        else {\n" +
+                     own_tile(true) + "        }\n    }\n";
+        }
+        else {
+            s += products("sc", "0", "    ") + "    __syncthreads();\n";
+            s += "    {\n        const int it = 0;\n" + iteration(tail != 0 ? partial : "0", true, tail != 0) + "    }\n";
+            if (steps > 1)
+                s += "    for (int it = 1; it < " + std::to_string(steps) + "; ++it) {\n" + iteration(whole("it"), false, false) + "    }\n";
+            s += gather(std::to_string((steps - 1) & 1), "    ");
+        }
 
         // what the split could not hold
-        s += "    sum += __shfl_xor(sum, 32, 64);\n    bool wrong = !(top <= PORCH_FLT_MAX) || !(sum > 0.0f && sum <= PORCH_FLT_MAX), small = false;\n";
+        s += "    sum += __shfl_xor(sum, 32, 64);\n";
+        if (split > 0) {
+            // the row's maximum and sum over all waves (a wave whose keys
+            // are all masked has a sum of 0)
+            s += "    if (lane < 32) {\n        maxima[wave][lane] = m;\n        sums[wave][lane] = sum;\n    }\n    __syncthreads();\n";
+            s += "    float row_max = maxima[0][lane & 31], row_sum = 0.0f;\n    #pragma unroll\n    for (int w = 1; w < " +
+                 std::to_string(waves) + "; ++w) row_max = __builtin_fmaxf(row_max, maxima[w][lane & 31]);\n";
+            s += "    #pragma unroll\n    for (int w = 0; w < " + std::to_string(waves) +
+                 "; ++w) row_sum += sums[w][lane & 31] * __builtin_amdgcn_exp2f(maxima[w][lane & 31] - row_max);\n";
+            s += "    float share = __builtin_amdgcn_exp2f(m - row_max);\n    sum = row_sum;\n";
+        }
+        s += "    bool wrong = !(top <= PORCH_FLT_MAX) || !(sum > 0.0f && sum <= PORCH_FLT_MAX), small = false;\n";
         s += "    #pragma unroll\n    for (int d = 0; d < " + DBS + "; ++d)\n        #pragma unroll\n        for (int v = 0; v < 16; ++v) {\n";
         s += "            const float x = __builtin_fabsf(acc[d][v]);\n";
         s += "            wrong |= !(x <= PORCH_FLT_MAX);\n            small |= !(x >= 0x1p-56f);\n        }\n";
@@ -472,7 +605,9 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
         // In fp32 throughout, in the order of the unfused program: every
         // row's maximum and sum first, then the weights, divided before they
         // meet V (undivided, large values could overflow).
+        // (Split keys: the first wave, with all of them.)
         s += "    if ((all & 1u) != 0 || (all & 6u) == 6u) {\n" + zero_acc;
+        if (split > 0) s += "        share = wave == 0 ? 1.0f : 0.0f;\n        if (wave == 0) {\n";
         s += "        m = -PORCH_FLT_MAX;\n        sum = 0.0f;\n";
         s += "        for (int pass = 0; pass < 2; ++pass) {\n        for (int key0 = 0; key0 < " + SK + "; key0 += 32) {\n";
         s += "            porch_v16f sc;\n            #pragma unroll\n            for (int v = 0; v < 16; ++v) sc[v] = 0.0f;\n";
@@ -494,16 +629,34 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
              " + (idx_t)porch_row_dim(d * 32 + (lane & 31)) * " + std::to_string(r.v.stride_col) + "] : 0.0f;\n";
         s += "                        acc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, sc[v], acc[d], 0, 0, 0);\n";
         s += "                    }\n            }\n        }\n";
-        s += "        if (pass == 0) sum += __shfl_xor(sum, 32, 64);\n        }\n        sum = 1.0f; // divided already\n    }\n";
+        s += "        if (pass == 0) sum += __shfl_xor(sum, 32, 64);\n        }\n";
+        if (split > 0) s += "        }\n";
+        s += "        sum = 1.0f; // divided already\n    }\n";
 
         // Output: register v of block d holds dim d 32 + 16 (v / 4 % 2) + 8 h +
         // 2 (v % 4) + v / 8: eight adjacent dims a lane from four registers of
         // either half of a block.
+        if (split > 0) {
+            s += "    #pragma unroll\n    for (int d = 0; d < " + DBS + "; ++d)\n        #pragma unroll\n        for (int v = 0; v < 16; ++v) parts[wave][d * 16 + v][lane] = acc[d][v] * share;\n";
+            s += "    __syncthreads();\n";
+        }
         s += "    if (own < " + SQ + ") {\n";
-        s += "        #pragma unroll\n        for (int d = 0; d < " + DBS + "; ++d)\n        #pragma unroll\n        for (int g = 0; g < 2; ++g) {\n";
+        if (split > 0) {
+            // the waves share the sums of their parts: 8 values a lane each
+            s += "        for (int u = wave; u < " + std::to_string(2 * DB) + "; u += " + std::to_string(waves) + ") {\n";
+            s += "            const int d = u >> 1, g = u & 1;\n";
+        }
+        else
+            s += "        #pragma unroll\n        for (int d = 0; d < " + DBS + "; ++d)\n        #pragma unroll\n        for (int g = 0; g < 2; ++g) {\n";
         s += "            float y[8];\n            const idx_t qn = d * 32 + 16 * g + 8 * h;\n";
         s += "            #pragma unroll\n            for (int e = 0; e < 8; ++e) {\n";
-        s += "                const float acc_v = acc[d][(e & 1) * 8 + 4 * g + (e >> 1)] / sum;\n";
+        if (split > 0) {
+            s += "                const int at = d * 16 + (e & 1) * 8 + 4 * g + (e >> 1);\n                float all_keys = parts[0][at][lane];\n";
+            s += "                #pragma unroll\n                for (int w = 1; w < " + std::to_string(waves) + "; ++w) all_keys += parts[w][at][lane];\n";
+            s += "                const float acc_v = all_keys / sum;\n";
+        }
+        else
+            s += "                const float acc_v = acc[d][(e & 1) * 8 + 4 * g + (e >> 1)] / sum;\n";
         s += "                const idx_t q1 = qn + e;\n                (void)q1;\n";
         {
             gemm_request e;

@@ -198,3 +198,43 @@ def test_layouts(gpu):
     for x, views in layouts(lambda a: gpu.tensor(list(a.shape), a.reshape(-1)), np.random.default_rng(5)):
         want, scale = reference(*x, 0.125)
         close(gpu.materialize(attention(*views, 0.125)).cpu().reshape(want.shape), want, scale)
+
+
+# (batch, queries, keys, dim, masked): past the blocks of 32 queries whose
+# keys are split over waves (512 of them, 256 at dim 128): the shared tiles
+SHARED = [(19, 865, 130, 64, True), (19, 865, 64, 32, False), (19, 865, 200, 32, True), (10, 831, 65, 128, False)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("size", SHARED + [(16, 1024, 40, 64, True), (8, 1024, 100, 128, True), (1, 32, 1000, 64, True)])
+def test_either_side_of_the_key_split(gpu, size):
+    q, k, v, mask = inputs(size, np.random.default_rng(6))
+    expr = graph(lambda x: gpu.tensor(list(x.shape), x.reshape(-1)), q, k, v, mask)
+    (kernel,) = gpu.plan(expr)["kernels"]
+    blocks = size[0] * -(-size[1] // 32)
+    assert (kernel["grid"][0] == blocks) == (size not in SHARED)
+    want, scale = reference(q, k, v, size[3] ** -0.5, mask)
+    close(gpu.materialize(expr).cpu().reshape(want.shape), want, scale)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", SPECIAL)
+def test_special_values_in_shared_tiles(gpu, name):
+    size = (19, 865, 70, 64, True)
+    q, k, v, mask = inputs(size, np.random.default_rng(7))
+    special(name, q, k, v, mask)
+    with np.errstate(invalid="ignore"):
+        want, scale = reference(q, k, v, 0.125, mask)
+    expr = graph(lambda x: gpu.tensor(list(x.shape), x.reshape(-1)), q, k, v, mask)
+    close(gpu.materialize(expr).cpu().reshape(want.shape), want, scale)
+
+
+@pytest.mark.gpu
+def test_keys_masked_to_minus_infinity_for_whole_waves(gpu):
+    # causal: most waves' keys weigh nothing for the first queries
+    size = (2, 256, 256, 64, True)
+    q, k, v, mask = inputs(size, np.random.default_rng(8))
+    mask[:] = np.where(np.tri(256, dtype=bool), np.float32(0), np.float32(-np.inf))
+    want, scale = reference(q, k, v, 0.125, mask)
+    expr = graph(lambda x: gpu.tensor(list(x.shape), x.reshape(-1)), q, k, v, mask)
+    close(gpu.materialize(expr).cpu().reshape(want.shape), want, scale)
