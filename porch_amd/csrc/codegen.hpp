@@ -247,8 +247,8 @@ namespace porch::cg {
         index_width width;
         int compute_units = 256;
     };
-    // dim of 32, 64 or 128, 32 rows and keys or more.
-    bool attention_fits(int64_t rows, int64_t keys, int64_t dim, int64_t value_dim);
+    // dim of 32, 64 or 128, 32 rows and keys or more, one launch's threads.
+    bool attention_fits(int64_t batch, int64_t rows, int64_t keys, int64_t dim, int64_t value_dim);
     kernel_code emit_attention(const attention_request& request);
 
     // A short K (8 to 64, a multiple of 8) over 256 columns or more, A's

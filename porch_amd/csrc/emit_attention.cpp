@@ -213,12 +213,14 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
 
     } // namespace
 
-    bool attention_fits(int64_t rows, int64_t keys, int64_t dim, int64_t value_dim) {
+    bool attention_fits(int64_t batch, int64_t rows, int64_t keys, int64_t dim, int64_t value_dim) {
+        // a launch holds fewer than 2^32 threads: 512 for 256 queries
+        if (batch * ((rows + 255) / 256) >= int64_t{1} << 23) return false;
         return dim == value_dim && (dim == 32 || dim == 64 || dim == 128) && rows >= 32 && keys >= 32;
     }
 
     kernel_code emit_attention(const attention_request& r) {
-        if (!attention_fits(r.rows, r.keys, r.dim, r.dim)) throw std::logic_error("emit_attention: shape");
+        if (!attention_fits(r.batch, r.rows, r.keys, r.dim, r.dim)) throw std::logic_error("emit_attention: shape");
         const int D = static_cast<int>(r.dim);
         // keys a tile: two buffers of K and V in 48 KB of LDS (96 at dim 128)
         const int KT = key_split(r) > 0 ? 32 : std::max(32, 2048 / D);

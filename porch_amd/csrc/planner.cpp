@@ -445,7 +445,7 @@ namespace porch::plan {
                 const std::vector<int64_t>& qs = g.at(first.lhs).out;
                 const std::vector<int64_t>& ks = g.at(first.rhs).out;
                 const std::vector<int64_t>& vs = g.at(second.rhs).out;
-                if (!cg::attention_fits(qs[o], ks[o + 1], qs[o + 1], vs[o + 1])) return false;
+                if (!cg::attention_fits(batched ? qs[0] : 1, qs[o], ks[o + 1], qs[o + 1], vs[o + 1])) return false;
                 // other reductions and products that f or the epilogue read
                 std::set<int> others;
                 boundaries(found.f, others, {found.qk}, true);

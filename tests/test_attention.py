@@ -130,6 +130,10 @@ def test_plans():
     # other head dimensions, fewer than 32 rows, another axis
     for shape in ([4, 128, 48], [4, 128, 256], [4, 20, 64]):
         assert "attention" not in kinds(attention(P(shape), P(shape), P(shape), 0.125))
+    # as many threads as a launch holds, and more
+    for batch, fused in (((1 << 23) - 1, True), (1 << 23, False)):
+        shape = [batch, 32, 32]
+        assert ("attention" in kinds(attention(P(shape), P(shape), P(shape), 0.125))) == fused
     s = porch.batched_matmul(q, porch.permute(k, [0, 2, 1]))
     assert "attention" not in kinds(porch.batched_matmul(porch.softmax(s, 1), v))
     # the weights or the scores are read elsewhere too
