@@ -37,10 +37,14 @@
 // the row's sum.  Weights reach the second product in 24 bits relative to the
 // row's maximum down to 2^-109 of it (smaller ones lose at most 2^-133).
 // Against 64 bits, normal q, k and v: 1.0e-6 (the unfused program: 1.2e-6).
-// What this cannot hold (values that are not finite anywhere, nonzero Q or K
-// below 2^-109, nonzero V below 2^-109 beside an output below 2^-56 or
-// operands of 2^30, rows whose scores are all below -2^100) sends the
-// workgroup to `redo`: fp32 MFMAs, in the unfused program's order.
+// What this cannot hold (values of 2^60 and more, infinities and NaN in any
+// operand, nonzero Q or K below 2^-109, nonzero V below 2^-109 beside an
+// output below 2^-56 or operands of 2^30, sums that are not finite, rows whose
+// scores are all below -2^100) sends the workgroup to `redo`: fp32 MFMAs, in
+// the unfused program's order.  The operands are what is looked at, not the
+// scores: below 2^60 no product over 128 dims leaves fp32's range, and a NaN
+// that a larger one makes in the split need not outlive f (a maximum or
+// minimum of NaN and a number is the number).
 
 #include "emit_gemm.hpp"
 
@@ -313,7 +317,7 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
             s += load_code(K, whole("1"), "", "    ") + store_code(K, "1", "    ");
             s += load_code(K, whole(steps > 2 ? "2" : "1"), "", "    ");
         }
-        s += "    float m = -0x1p100f, sum = 0.0f, top = 0.0f, al = 1.0f;\n    (void)al;\n    porch_v16f acc[" + DBS + "], sc[" + KBS + "];\n    porch_b8 pf[" + std::to_string(KT / 16) + "][3];\n";
+        s += "    float m = -0x1p100f, sum = 0.0f, al = 1.0f;\n    (void)al;\n    porch_v16f acc[" + DBS + "], sc[" + KBS + "];\n    porch_b8 pf[" + std::to_string(KT / 16) + "][3];\n";
         const std::string zero_acc = "    #pragma unroll\n    for (int d = 0; d < " + DBS +
                                      "; ++d)\n        #pragma unroll\n        for (int v = 0; v < 16; ++v) acc[d][v] = 0.0f;\n";
         s += zero_acc;
@@ -417,7 +421,6 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
         auto weights = [&](const std::string& key0, bool masked, const std::string& pf, const std::string& ind) {
             std::string c;
             c += ind + "#pragma unroll\n" + ind + "for (int b = 0; b < " + KBS + "; ++b) {\n";
-            c += ind + "    #pragma unroll\n" + ind + "    for (int v = 0; v < 16; ++v) top = __builtin_fmaxf(top, __builtin_fabsf(sc[b][v]));\n";
             c += scores("sc[b]", "(idx_t)(" + key0 + ") + b * 32", masked, ind + "    ");
             c += ind + "}\n";
             c += ind + "float tm = sc[0][0];\n";
@@ -595,7 +598,7 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
                  "; ++w) row_sum += sums[w][lane & 31] * __builtin_amdgcn_exp2f(maxima[w][lane & 31] - row_max);\n";
             s += "    float share = __builtin_amdgcn_exp2f(m - row_max);\n    sum = row_sum;\n";
         }
-        s += "    bool wrong = !(top <= PORCH_FLT_MAX) || !(sum > 0.0f && sum <= PORCH_FLT_MAX), small = false;\n";
+        s += "    bool wrong = largest.x >= 0x5d80 || largest.y >= 0x5d80 || !(sum > 0.0f && sum <= PORCH_FLT_MAX), small = false;\n";
         s += "    #pragma unroll\n    for (int d = 0; d < " + DBS + "; ++d)\n        #pragma unroll\n        for (int v = 0; v < 16; ++v) {\n";
         s += "            const float x = __builtin_fabsf(acc[d][v]);\n";
         s += "            wrong |= !(x <= PORCH_FLT_MAX);\n            small |= !(x >= 0x1p-56f);\n        }\n";

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 import porch_amd as porch
+from oracle import host
 from tests.helpers import placeholder
 from tests.kernel_emu import emulate as emu
 
@@ -242,3 +243,80 @@ def test_keys_masked_to_minus_infinity_for_whole_waves(gpu):
     want, scale = reference(q, k, v, 0.125, mask)
     expr = graph(lambda x: gpu.tensor(list(x.shape), x.reshape(-1)), q, k, v, mask)
     close(gpu.materialize(expr).cpu().reshape(want.shape), want, scale)
+
+
+# Products that the split cannot form, under a score function that gives a
+# number for NaN (a > b ? a : b): the score is f of the fp32 product.
+FUNCTIONS = {"relu": porch.relu, "at most 4": lambda s: porch.minimum(s, 4.0), "at least -4": lambda s: porch.maximum(s, -4.0)}
+PRODUCTS = ["key past bf16", "query past bf16", "infinite key", "infinite query", "nan key", "products past fp32"]
+
+
+def product_inputs(name, size, rng):
+    q, k, v, _ = inputs((*size, False), rng)
+    tiny = lambda n: (rng.uniform(0.5, 1.0, n) * rng.choice([-1.0, 1.0], n)).astype(np.float32) * np.float32(1e-31)
+    if name == "key past bf16":
+        q[0, :, 3] = tiny(size[1])
+        k[0, 5, 3] = np.float32(3.4e38)
+    elif name == "query past bf16":
+        q[0, 2, 3] = np.float32(3.4e38)
+        k[0, :, 3] = tiny(size[2])
+    elif name == "infinite key":
+        k[0, 5, 3] = -np.inf
+    elif name == "infinite query":
+        q[0, 2, 3] = np.inf
+    elif name == "nan key":
+        k[0, 5, 3] = np.nan
+    else:
+        q[0, 2, 3:5] = np.float32(1e30)
+        k[0, 5, 3] = np.float32(1e30)
+        k[0, 6, 3] = np.float32(-1e30)
+        k[0, 7, 3:5] = np.float32([1e30, -1e30])
+    return q, k, v
+
+
+def product_graph(make, q, k, v, f):
+    scores = FUNCTIONS[f](porch.batched_matmul(make(q), porch.permute(make(k), [0, 2, 1])) * 0.125)
+    return porch.batched_matmul(porch.softmax(scores, 2), make(v))
+
+
+def check_products(got, expr, v):
+    want = host.evaluate(expr).reshape(got.shape)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    ok = ~np.isnan(want)
+    # as in close(), with the weights' sum of 1 bounding the scale
+    assert np.all(np.abs(got[ok].astype(np.float64) - want[ok]) <= 64 * 2.0 ** -23 * np.abs(v).max())
+
+
+@pytest.mark.skipif(not emu.available(), reason="no clang for the emulation")
+@pytest.mark.parametrize("name", PRODUCTS)
+def test_emulated_products_hidden_by_the_scores(name):
+    for f in ("relu", "at most 4"):
+        q, k, v = product_inputs(name, (1, 33, 40, 64), np.random.default_rng(11))
+        expr = product_graph(host_only, q, k, v, f)
+        assert kinds(expr) == ["attention"]
+        got = emu.evaluate(expr, [q, k, v], timeout=300)
+        check_products(got.reshape(v.shape[0], -1, v.shape[2]), expr, v)
+
+
+@pytest.mark.skipif(not emu.available(), reason="no clang for the emulation")
+def test_emulated_products_hidden_by_the_scores_in_shared_tiles():
+    for name in ("key past bf16", "products past fp32"):
+        q, k, v = product_inputs(name, (19, 865, 70, 64), np.random.default_rng(12))
+        expr = product_graph(host_only, q, k, v, "relu")
+        (kernel,) = porch.plan(expr)["kernels"]
+        assert kernel["kind"] == "attention" and kernel["grid"][0] < 19 * 28
+        got = emu.evaluate(expr, [q, k, v], timeout=300, only=[0])
+        rows = kernel["block"] // 2  # 32 queries a wave
+        got = got.reshape(v.shape[0], -1, v.shape[2])[:1, :rows]
+        check_products(got, product_graph(host_only, q[:1, :rows], k[:1], v[:1], "relu"), v)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("f", sorted(FUNCTIONS))
+@pytest.mark.parametrize("name", PRODUCTS)
+def test_products_hidden_by_the_scores(gpu, name, f):
+    for size in [(1, 33, 40, 64), (19, 865, 70, 64), (19, 865, 70, 32)]:
+        q, k, v = product_inputs(name, size, np.random.default_rng(13))
+        expr = product_graph(lambda x: gpu.tensor(list(x.shape), x.reshape(-1)), q, k, v, f)
+        assert kinds(expr) == ["attention"]
+        check_products(gpu.materialize(expr).cpu().reshape(v.shape[0], size[1], size[3]), expr, v)
