@@ -32,15 +32,18 @@
 // products of the split make that 1.2 PFLOP/s of bf16, against the 1.34-1.42
 // that this card's large bf16 products reach.
 //
-// Accuracy: a weight is exp2(s log2 e - M) with M the running maximum of
-// s log2 e: one rounding, and whatever M's own rounding is cancels against
-// the row's sum.  Weights reach the second product in 24 bits relative to the
-// row's maximum down to 2^-109 of it (smaller ones lose at most 2^-133).
+// Accuracy: a weight is exp2((s - m) log2 e) with m the running maximum of s,
+// so that a row's largest weight is 1 whatever its scores' size.  (One
+// instruction a score less, exp2(fma(s, log2 e, -M)) with M = m log2 e
+// rounded, leaves M's rounding in every weight: from scores of 2^31 on the
+// largest weight of a row can be 2^-128, where the split keeps four bits.)
+// Weights reach the second product in 24 bits relative to the row's maximum
+// down to 2^-109 of it (smaller ones lose at most 2^-133).
 // Against 64 bits, normal q, k and v: 1.0e-6 (the unfused program: 1.2e-6).
 // What this cannot hold (values of 2^60 and more, infinities and NaN in any
 // operand, nonzero Q or K below 2^-109, nonzero V below 2^-109 beside an
 // output below 2^-56 or operands of 2^30, sums that are not finite, rows whose
-// scores are all below -2^100) sends the workgroup to `redo`: fp32 MFMAs, in
+// scores are all -inf) sends the workgroup to `redo`: fp32 MFMAs, in
 // the unfused program's order.  The operands are what is looked at, not the
 // scores: below 2^60 no product over 128 dims leaves fp32's range, and a NaN
 // that a larger one makes in the split need not outlive f (a maximum or
@@ -317,7 +320,7 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
             s += load_code(K, whole("1"), "", "    ") + store_code(K, "1", "    ");
             s += load_code(K, whole(steps > 2 ? "2" : "1"), "", "    ");
         }
-        s += "    float m = -0x1p100f, sum = 0.0f, al = 1.0f;\n    (void)al;\n    porch_v16f acc[" + DBS + "], sc[" + KBS + "];\n    porch_b8 pf[" + std::to_string(KT / 16) + "][3];\n";
+        s += "    float m = -PORCH_FLT_MAX, sum = 0.0f, al = 1.0f;\n    (void)al;\n    porch_v16f acc[" + DBS + "], sc[" + KBS + "];\n    porch_b8 pf[" + std::to_string(KT / 16) + "][3];\n";
         const std::string zero_acc = "    #pragma unroll\n    for (int d = 0; d < " + DBS +
                                      "; ++d)\n        #pragma unroll\n        for (int v = 0; v < 16; ++v) acc[d][v] = 0.0f;\n";
         s += zero_acc;
@@ -427,11 +430,11 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
             c += ind + "#pragma unroll\n" + ind + "for (int b = 0; b < " + KBS + "; ++b)\n" + ind + "    #pragma unroll\n" + ind +
                  "    for (int v = 0; v < 16; ++v) tm = __builtin_fmaxf(tm, sc[b][v]);\n";
             c += ind + "tm = __builtin_fmaxf(tm, __shfl_xor(tm, 32, 64));\n";
-            c += ind + "const float ml = __builtin_fmaxf(m, tm * 0x1.715476p+0f);\n";
-            c += ind + "const float alpha = __builtin_amdgcn_exp2f(m - ml);\n" + ind + "m = ml;\n";
+            c += ind + "const float mn = __builtin_fmaxf(m, tm);\n";
+            c += ind + "const float alpha = __builtin_amdgcn_exp2f((m - mn) * 0x1.715476p+0f);\n" + ind + "m = mn;\n";
             c += ind + "float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};\n";
             c += ind + "#pragma unroll\n" + ind + "for (int b = 0; b < " + KBS + "; ++b)\n" + ind + "    #pragma unroll\n" + ind +
-                 "    for (int v = 0; v < 16; ++v) {\n" + ind + "        sc[b][v] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[b][v], 0x1.715476p+0f, -m));\n" + ind +
+                 "    for (int v = 0; v < 16; ++v) {\n" + ind + "        sc[b][v] = __builtin_amdgcn_exp2f((sc[b][v] - m) * 0x1.715476p+0f);\n" + ind +
                  "        part[v & 3] += sc[b][v];\n" + ind + "    }\n";
             c += ind + "sum = sum * alpha + ((part[0] + part[1]) + (part[2] + part[3]));\n";
             c += ind + "#pragma unroll\n" + ind + "for (int t = 0; t < " + std::to_string(KT / 16) + "; ++t) {\n";
@@ -595,8 +598,8 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
             s += "    float row_max = maxima[0][lane & 31], row_sum = 0.0f;\n    #pragma unroll\n    for (int w = 1; w < " +
                  std::to_string(waves) + "; ++w) row_max = __builtin_fmaxf(row_max, maxima[w][lane & 31]);\n";
             s += "    #pragma unroll\n    for (int w = 0; w < " + std::to_string(waves) +
-                 "; ++w) row_sum += sums[w][lane & 31] * __builtin_amdgcn_exp2f(maxima[w][lane & 31] - row_max);\n";
-            s += "    float share = __builtin_amdgcn_exp2f(m - row_max);\n    sum = row_sum;\n";
+                 "; ++w) row_sum += sums[w][lane & 31] * __builtin_amdgcn_exp2f((maxima[w][lane & 31] - row_max) * 0x1.715476p+0f);\n";
+            s += "    float share = __builtin_amdgcn_exp2f((m - row_max) * 0x1.715476p+0f);\n    sum = row_sum;\n";
         }
         s += "    bool wrong = largest.x >= 0x5d80 || largest.y >= 0x5d80 || !(sum > 0.0f && sum <= PORCH_FLT_MAX), small = false;\n";
         s += "    #pragma unroll\n    for (int d = 0; d < " + DBS + "; ++d)\n        #pragma unroll\n        for (int v = 0; v < 16; ++v) {\n";

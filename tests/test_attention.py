@@ -320,3 +320,37 @@ def test_products_hidden_by_the_scores(gpu, name, f):
         expr = product_graph(lambda x: gpu.tensor(list(x.shape), x.reshape(-1)), q, k, v, f)
         assert kinds(expr) == ["attention"]
         check_products(gpu.materialize(expr).cpu().reshape(v.shape[0], size[1], size[3]), expr, v)
+
+
+# Whole rows masked with a finite value: their scores are that value (it
+# absorbs them), their weights equal.  fp32 values of 2^31 and more lie 256
+# and more apart, 2^369 in weights.  One value per entry: nothing else sends
+# its workgroups to the fp32 MFMAs.
+MASKS = [-1e9, -4.1e9, -1.26e10, -2.21e10, 4.1e9, -6e9, -3.4028235e38]
+
+
+def masked_rows_graph(make, size, seed):
+    q, k, v, _ = inputs((*size, False), np.random.default_rng(seed))
+    mask = np.zeros((size[0], size[1], size[2]), np.float32)
+    for i, x in enumerate(MASKS):
+        mask[i, 0] = x          # the row
+        mask[i, 1, 1::2] = x    # half of its keys
+        mask[i, 2, 33:] = x     # the keys behind the first tile
+        mask[i, 3, :33] = x     # and those of the first
+    return (q, k, mask, v), graph(make, q, k, v, mask)
+
+
+@pytest.mark.skipif(not emu.available(), reason="no clang for the emulation")
+def test_emulated_rows_masked_with_finite_values():
+    values, expr = masked_rows_graph(host_only, (len(MASKS), 32, 50, 64), 14)
+    assert kinds(expr) == ["attention"]
+    check_products(emu.evaluate(expr, values, timeout=300), expr, values[3])
+
+
+@pytest.mark.gpu
+def test_rows_masked_with_finite_values(gpu):
+    for size in [(7, 32, 50, 64), (7, 100, 300, 64), (19, 865, 70, 64), (19, 865, 130, 32), (10, 831, 65, 128)]:
+        values, expr = masked_rows_graph(lambda x: gpu.tensor(list(x.shape), x.reshape(-1)), size, 15)
+        assert kinds(expr) == ["attention"]
+        got = gpu.materialize(expr).cpu().reshape(size[0], size[1], size[3])
+        check_products(got, expr, values[3])
