@@ -38,16 +38,18 @@
 // rounded, leaves M's rounding in every weight: from scores of 2^31 on the
 // largest weight of a row can be 2^-128, where the split keeps four bits.)
 // Weights reach the second product in 24 bits relative to the row's maximum
-// down to 2^-109 of it (smaller ones lose at most 2^-133).
+// down to 2^-109 of it; smaller ones lose at most 2^-133, and those below
+// 2^-126, which the hardware's exp2 makes zero, all.  With values of V below
+// 2^30 that moves an output by at most 2^-96 a key.
 // Against 64 bits, normal q, k and v: 1.0e-6 (the unfused program: 1.2e-6).
-// What this cannot hold (values of 2^60 and more, infinities and NaN in any
+// What this cannot hold (values of 2^30 and more, infinities and NaN in any
 // operand, nonzero Q or K below 2^-109, nonzero V below 2^-109 beside an
-// output below 2^-56 or operands of 2^30, sums that are not finite, rows whose
-// scores are all -inf) sends the workgroup to `redo`: fp32 MFMAs, in
-// the unfused program's order.  The operands are what is looked at, not the
-// scores: below 2^60 no product over 128 dims leaves fp32's range, and a NaN
-// that a larger one makes in the split need not outlive f (a maximum or
-// minimum of NaN and a number is the number).
+// output below 2^-56, sums that are not finite, rows whose scores are all
+// -inf) sends the workgroup to `redo`: fp32 MFMAs, in the unfused program's
+// order.  The operands are what is looked at, not the scores: below 2^30 no
+// product over 128 dims leaves fp32's range, and a NaN that a larger value
+// makes in the split need not outlive f (a maximum or minimum of NaN and a
+// number is the number).
 
 #include "emit_gemm.hpp"
 
@@ -601,12 +603,12 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
                  "; ++w) row_sum += sums[w][lane & 31] * __builtin_amdgcn_exp2f((maxima[w][lane & 31] - row_max) * 0x1.715476p+0f);\n";
             s += "    float share = __builtin_amdgcn_exp2f((m - row_max) * 0x1.715476p+0f);\n    sum = row_sum;\n";
         }
-        s += "    bool wrong = largest.x >= 0x5d80 || largest.y >= 0x5d80 || !(sum > 0.0f && sum <= PORCH_FLT_MAX), small = false;\n";
+        s += "    bool wrong = largest.x >= 0x4e80 || largest.y >= 0x4e80 || !(sum > 0.0f && sum <= PORCH_FLT_MAX), small = false;\n";
         s += "    #pragma unroll\n    for (int d = 0; d < " + DBS + "; ++d)\n        #pragma unroll\n        for (int v = 0; v < 16; ++v) {\n";
         s += "            const float x = __builtin_fabsf(acc[d][v]);\n";
         s += "            wrong |= !(x <= PORCH_FLT_MAX);\n            small |= !(x >= 0x1p-56f);\n        }\n";
         s += "    const unsigned found = (__ballot(wrong || lowestK < 0x12000000u) != 0 ? 1u : 0u) |\n"
-             "                           (__ballot(small || largest.x >= 0x4e80 || largest.y >= 0x4e80) != 0 ? 2u : 0u) |\n"
+             "                           (__ballot(small) != 0 ? 2u : 0u) |\n"
              "                           (__ballot(lowestV < 0x12000000u) != 0 ? 4u : 0u);\n";
         s += "    if (lane == 0) seen[wave] = found;\n    __syncthreads();\n";
         s += "    unsigned all = 0;\n    #pragma unroll\n    for (int w = 0; w < " + std::to_string(waves) + "; ++w) all |= seen[w];\n";

@@ -201,7 +201,12 @@ namespace emu {
 #define __shfl(v, s, w) emu::shfl((v), (s), (w))
 #define __ballot(p) emu::ballot(p)
 #define __builtin_amdgcn_rcpf(x) (1.0f / (x))
-#define __builtin_amdgcn_exp2f(x) exp2f(x)
+// v_exp_f32: results below the least normal value come out as zero
+static inline float porch_emu_exp2(float x) {
+    const float r = exp2f(x);
+    return r < 0x1p-126f ? 0.0f : r;
+}
+#define __builtin_amdgcn_exp2f(x) porch_emu_exp2(x)
 #define __builtin_amdgcn_sched_group_barrier(a, b, c) ((void)0)
 #define __builtin_amdgcn_sched_barrier(a) ((void)0)
 #define __builtin_amdgcn_wave_barrier() emu::wave_sync()

@@ -354,3 +354,39 @@ def test_rows_masked_with_finite_values(gpu):
         assert kinds(expr) == ["attention"]
         got = gpu.materialize(expr).cpu().reshape(size[0], size[1], size[3])
         check_products(got, expr, values[3])
+
+
+def faint_inputs(size, value, seed):
+    """The first key has the largest score of every query, 88 to 94 above the
+    others': V is zero there, and `value` at two keys of weights around 2^-130."""
+    rng = np.random.default_rng(seed)
+    q, k, v, _ = inputs((*size, False), rng)
+    q[:], k[:], v[:] = 0, 0, 0
+    q[:, :, 0] = rng.uniform(28.0, 30.0, q.shape[:2])
+    k[:, 0, 0] = 3.125 * size[3] ** 0.5
+    v[:, 3, 5] = value
+    v[:, size[2] - 2, 7] = -value
+    return q, k, v
+
+
+def check_faint(got, q, k, v):
+    want, scale = reference(q, k, v, q.shape[2] ** -0.5)
+    # a denormal weight's last bit, 2^-149, on top of close()'s
+    assert np.all(np.abs(got - want) <= 64 * 2.0 ** -23 * scale + 2.0 ** -148 * np.abs(v).max())
+    assert np.all(got[:, :, 5] != 0) and np.all(got[:, :, 7] != 0)
+
+
+@pytest.mark.skipif(not emu.available(), reason="no clang for the emulation")
+def test_emulated_faint_weights_of_large_values():
+    for value in (2.0 ** 31, 2.0 ** 100):
+        q, k, v = faint_inputs((1, 32, 70, 64), np.float32(value), 16)
+        check_faint(emulated(q, k, v, None), q, k, v)
+
+
+@pytest.mark.gpu
+def test_faint_weights_of_large_values(gpu):
+    for value in (2.0 ** 31, 2.0 ** 100):
+        for size in [(1, 32, 70, 64), (19, 865, 70, 64), (19, 865, 130, 32)]:
+            q, k, v = faint_inputs(size, np.float32(value), 17)
+            expr = graph(lambda x: gpu.tensor(list(x.shape), x.reshape(-1)), q, k, v, None)
+            check_faint(gpu.materialize(expr).cpu().reshape(q.shape), q, k, v)
