@@ -4,9 +4,9 @@
 // (reference src/tensor.cpp:684-721).  Here small products use the same
 // one-output-per-lane K loop (sequential fp32 sum, exactly the reference's
 // order), and large ones the matrix cores: three bf16 values per fp32 one
-// (emit_gemm_split.cpp), or for many tiles of a short K the persistent fp32
-// MFMA kernel below.  A batched product runs the same kernels over (batch entry, tile) pairs, each entry's operands
-// offset by their batch strides.
+// (emit_gemm_split.cpp), or for a short K the fp32 MFMA kernels below.  A
+// batched product runs the same kernels over (batch entry, tile) pairs, each
+// entry's operands offset by their batch strides.
 
 #include "emit_gemm.hpp"
 
@@ -88,9 +88,9 @@ namespace porch::cg {
         }
 
         // ----------------------------------------------------------------
-        // LDS-tiled fp32 MFMA over a short K: 128x128 tiles per 256-thread
-        // workgroup, each
-        // wave a 64x64 quadrant as 2x2 v_mfma_f32_32x32x2f32 blocks, K in
+        // LDS-tiled fp32 MFMA over a short K: 128x128 tile per 256-thread
+        // workgroup, each wave a 64x64 quadrant as 2x2
+        // v_mfma_f32_32x32x2f32 blocks, K in
         // steps of 16 through double-buffered LDS (one barrier per step).
         // Operand lane layout (checked on gfx950): A[i = l%32][k = l/32],
         // B[k = l/32][j = l%32]; accumulator register v of lane l holds
@@ -228,12 +228,12 @@ namespace porch::cg {
 
         // LDS stores of the next K-slice per wave, and whether they and the
         // global loads fit between a step's MFMAs
-        int ds_writes_of(const operand_layout& la, const operand_layout& lb) {
-            return (la.k_major ? 2 : 4) * (BM / 64) + (lb.k_major ? 2 : 4) * (BN / 64);
+        int ds_writes_of(const operand_layout& la, const operand_layout& lb, int rows) {
+            return (la.k_major ? 2 : 4) * (rows / 64) + (lb.k_major ? 2 : 4) * (BN / 64);
         }
-        bool interleaves(const operand_layout& la, const operand_layout& lb) {
+        bool interleaves(const operand_layout& la, const operand_layout& lb, int rows) {
             return la.vector && lb.vector &&
-                   4 * (BM / 64 + BN / 64) + 4 + ds_writes_of(la, lb) <= (BK / 2) * (BM / 64) * 2;
+                   4 * (rows / 64 + BN / 64) + 4 + ds_writes_of(la, lb, rows) <= (BK / 2) * (rows / 64) * 2;
         }
 
         // A short K (at most 4 steps, K <= 64) with more tiles than
@@ -250,34 +250,44 @@ namespace porch::cg {
         // branch-free.  Two accumulator sets need 128-row tiles (a wave's
         // 64 x 64 block) to stay within the register budget of two
         // workgroups per compute unit.
-        bool persistent(const gemm_request& r) {
+        bool fp32_persistent(const gemm_request& r) {
             const int64_t tiles = ((r.m + BM - 1) / BM) * ((r.n + BN - 1) / BN) * r.batch;
             return r.k_chunks == 1 && r.k <= 4 * BK && tiles > static_cast<int64_t>(std::max(r.compute_units, 1)) * 2 &&
                    r.batch * r.m * r.n < (int64_t{1} << 29) &&
-                   interleaves(layout_of(r.a, true, r.m, r.k), layout_of(r.b, false, r.n, r.k));
+                   interleaves(layout_of(r.a, true, r.m, r.k), layout_of(r.b, false, r.n, r.k), BM);
         }
 
-        kernel_code emit_gemm_persistent(const gemm_request& r) {
+        kernel_code emit_gemm_fp32(const gemm_request& r) {
             const int64_t tiles_n = (r.n + BN - 1) / BN;
             const int64_t steps = (r.k + BK - 1) / BK;
             const operand_layout la = layout_of(r.a, true, r.m, r.k);
             const operand_layout lb = layout_of(r.b, false, r.n, r.k);
+            const bool scheduled = la.vector && lb.vector;
             const int64_t resident = static_cast<int64_t>(std::max(r.compute_units, 1)) * 2;
             const int64_t out_elems = r.batch * r.m * r.n;
-            const int ib = BM / 64; // 32-row MFMA blocks per wave
-            const int64_t tiles = ((r.m + BM - 1) / BM) * tiles_n;
+            const bool persistent = fp32_persistent(r);
+            // Otherwise 256-row tiles (each wave 128 x 64: 4 x 2 MFMA blocks)
+            // halve the LDS reads per MFMA and the B re-reads; used while
+            // they still give every compute unit a tile.
+            const int bm = persistent ? BM
+                           : (r.m >= 256 && ((r.m + 255) / 256) * tiles_n * r.batch >= r.compute_units) ? 256
+                                                                                                        : BM;
+            const int ib = bm / 64; // 32-row MFMA blocks per wave
+            const int64_t tiles_m = (r.m + bm - 1) / bm;
+            const int64_t tiles = tiles_m * tiles_n;
             const int64_t total = tiles * r.batch; // (batch entry, tile) pairs
             const std::string IB = std::to_string(ib);
-            const std::string HALF = std::to_string(BM / 2);
-            const int vmem = BM / 64 + BN / 64;
+            const std::string HALF = std::to_string(bm / 2);
+            const int vmem = bm / 64 + BN / 64;
             const int mfmas = (BK / 2) * ib * 2;
-            const int ds_writes = ds_writes_of(la, lb);
+            const int ds_writes = ds_writes_of(la, lb, bm);
+            const bool interleave = interleaves(la, lb, bm);
             kernel_code kc;
             kc.kind = "gemm.mfma";
             kc.name = "porch_gemm";
             kc.n_slots = r.n_slots;
             kc.block = 256;
-            kc.grid_x = static_cast<unsigned>(resident);
+            kc.grid_x = static_cast<unsigned>(persistent ? resident : total);
             const char* T = r.width.type();
             std::string& s = kc.source;
             s = kernel_prologue(r.n_slots, T);
@@ -286,7 +296,7 @@ namespace porch::cg {
             // register budget within which the accumulators stay in VGPRs.
             s += "extern \"C\" __global__ void __launch_bounds__(256, 2) porch_gemm(" +
                  kernel_params(r.n_slots) + ") {\n";
-            s += "    __shared__ __attribute__((aligned(16))) float As[2][2][" + std::to_string(BM) + "][" +
+            s += "    __shared__ __attribute__((aligned(16))) float As[2][2][" + std::to_string(bm) + "][" +
                  std::to_string(PITCH) + "];\n";
             s += "    __shared__ __attribute__((aligned(16))) float Bs[2][2][" + std::to_string(BN) + "][" +
                  std::to_string(PITCH) + "];\n";
@@ -298,7 +308,8 @@ namespace porch::cg {
             // each XCD a contiguous band of tile rows so its L2 holds them.
             // (For a batched product the bands run over (entry, tile) pairs,
             // entry-major, so an XCD holds whole entries where it can.)
-            // Tile `raw` (a workgroup's running index) -> m0, n0 (and qb), A, B with name suffix `sx`.
+            // Tile `raw` (a workgroup index, or a persistent workgroup's
+            // running index) -> m0, n0 (and qb), A, B with name suffix `sx`.
             // With a grid that is a multiple of 8, raw % 8 is the XCD.
             auto decode = [&](const std::string& raw, const std::string& sx, const std::string& ind) {
                 std::string d;
@@ -315,7 +326,7 @@ namespace porch::cg {
                     d += ind + "const int tile" + sx + " = " + lin + " % " + std::to_string(tiles) + ";\n";
                 }
                 d += ind + "const idx_t m0" + sx + " = (idx_t)(tile" + sx + " / " + std::to_string(tiles_n) +
-                     ") * " + std::to_string(BM) + ";\n";
+                     ") * " + std::to_string(bm) + ";\n";
                 d += ind + "const idx_t n0" + sx + " = (idx_t)(tile" + sx + " % " + std::to_string(tiles_n) +
                      ") * " + std::to_string(BN) + ";\n";
                 auto base = [&](const gemm_operand& op) {
@@ -328,11 +339,12 @@ namespace porch::cg {
                 d += ind + "const float* __restrict__ B" + sx + " = " + base(r.b) + ";\n";
                 return d;
             };
+            if (!persistent) s += decode("blockIdx.x", "", "    ");
             // Even step counts of a persistent kernel load two K-slices
             // ahead, through two register sets: a slice's LDS store then
             // waits only for loads issued a step earlier, behind the output
             // stores of two steps before, not of the step before.
-            const bool ahead2 = steps % 2 == 0;
+            const bool ahead2 = persistent && steps % 2 == 0;
             auto in_set = [](std::string code, int set) {
                 for (const char* name : {"rA[", "rB["}) {
                     const std::string from{name};
@@ -344,21 +356,22 @@ namespace porch::cg {
             };
             if (ahead2)
                 for (int set = 0; set < 2; ++set)
-                    s += "    float rA" + std::to_string(set) + "[" + std::to_string(4 * (BM / 64)) + "];\n    float rB" +
+                    s += "    float rA" + std::to_string(set) + "[" + std::to_string(4 * (bm / 64)) + "];\n    float rB" +
                          std::to_string(set) + "[8];\n";
             else
-                s += "    float rA[" + std::to_string(4 * (BM / 64)) + "];\n    float rB[8];\n";
+                s += "    float rA[" + std::to_string(4 * (bm / 64)) + "];\n    float rB[8];\n";
             s += "    floatx16 acc[" + IB + "][2];\n";
             const std::string zero_acc =
                 "    #pragma unroll\n    for (int i = 0; i < " + IB + "; ++i)\n"
                 "        #pragma unroll\n        for (int j = 0; j < 2; ++j)\n"
                 "            #pragma unroll\n            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;\n";
             std::string load_a, store_a, load_b, store_b;
-            operand_code(load_a, store_a, "A", r.a, true, r.m, r.k, la, BM);
+            operand_code(load_a, store_a, "A", r.a, true, r.m, r.k, la, bm);
             operand_code(load_b, store_b, "B", r.b, false, r.n, r.k, lb, BN);
+            if (!persistent) s += zero_acc;
             // prologue: the first K-slice of the (first) tile
             s += "    {\n";
-            s += decode("blockIdx.x", "", "        ");
+            if (persistent) s += decode("blockIdx.x", "", "        ");
             s += "        const idx_t k0 = 0;\n        const int nb = 0;\n";
             if (ahead2) {
                 s += in_set(load_a + load_b + store_a + store_b, 0);
@@ -371,68 +384,117 @@ namespace porch::cg {
             }
             s += "    }\n    __syncthreads();\n";
             // Epilogue for the accumulator blocks u = 2 bi + bj in [lo, hi)
-            // of `accP` at tile origin (m0p, n0p, qbp): branch-free, with
-            // clamped coordinates for the epilogue's own loads and the store
-            // offset set out of the buffer's range for lanes outside the
-            // output.
-            auto epilogue = [&](int lo, int hi) {
+            // of `accn` at tile origin (m0n, n0n, qbn).  Buffered: branch-free,
+            // with clamped coordinates for the epilogue's own loads and the
+            // store offset set out of the buffer's range for lanes outside
+            // the output.
+            auto epilogue = [&](const std::string& accn, const std::string& m0n, const std::string& n0n,
+                                const std::string& qbn, int lo, int hi, bool buffered) {
                 std::string e;
                 if (lo >= hi) return e;
                 const std::string M = std::to_string(r.m), N = std::to_string(r.n);
-                e += "    #pragma unroll\n    for (int u = " + std::to_string(lo) + "; u < " + std::to_string(hi) + "; ++u)\n";
-                e += "    #pragma unroll\n    for (int v = 0; v < 16; ++v) {\n";
-                e += "        const int bi = u >> 1;\n        const int bj = u & 1;\n";
-                e += "        const idx_t q0 = m0p + wm * " + HALF + " + bi * 32 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);\n";
-                e += "        const idx_t q1 = n0p + wn * 64 + bj * 32 + (lane & 31);\n";
-                e += "        const bool inb = q0 < " + M + " && q1 < " + N + ";\n";
-                e += "        const idx_t e0 = inb ? q0 : (idx_t)0;\n";
-                e += "        const idx_t e1 = inb ? q1 : (idx_t)0;\n";
-                e += "        const float acc_v = accP[bi][bj][v];\n";
+                if (buffered) {
+                    e += "    #pragma unroll\n    for (int u = " + std::to_string(lo) + "; u < " + std::to_string(hi) +
+                         "; ++u)\n";
+                    e += "    #pragma unroll\n    for (int v = 0; v < 16; ++v) {\n";
+                    e += "        const int bi = u >> 1;\n        const int bj = u & 1;\n";
+                }
+                else {
+                    e += "    #pragma unroll\n    for (int bi = 0; bi < " + IB + "; ++bi)\n";
+                    e += "    #pragma unroll\n    for (int bj = 0; bj < 2; ++bj)\n";
+                    e += "    #pragma unroll\n    for (int v = 0; v < 16; ++v) {\n";
+                }
+                e += "        const idx_t q0 = " + m0n + " + wm * " + HALF +
+                     " + bi * 32 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);\n";
+                e += "        const idx_t q1 = " + n0n + " + wn * 64 + bj * 32 + (lane & 31);\n";
                 std::string body;
                 emitter em(*r.expr, body, 1);
-                em.indent = "        ";
+                std::vector<std::string> names;
+                if (buffered) {
+                    e += "        const bool inb = q0 < " + M + " && q1 < " + N + ";\n";
+                    e += "        const idx_t e0 = inb ? q0 : (idx_t)0;\n";
+                    e += "        const idx_t e1 = inb ? q1 : (idx_t)0;\n";
+                    e += "        const float acc_v = " + accn + "[bi][bj][v];\n";
+                    em.indent = "        ";
+                    names = r.batched ? std::vector<std::string>{qbn, "e0", "e1"}
+                                      : std::vector<std::string>{"e0", "e1"};
+                }
+                else {
+                    e += "        if (q0 < " + M + " && q1 < " + N + ") {\n";
+                    e += "            const float acc_v = " + accn + "[bi][bj][v];\n";
+                    em.indent = "            ";
+                    names = r.batched ? std::vector<std::string>{qbn, "q0", "q1"}
+                                      : std::vector<std::string>{"q0", "q1"};
+                }
                 em.declare_roots({r.epilogue});
-                epilogue_emitter(em, r,
-                                 r.batched ? std::vector<std::string>{"qbp", "e0", "e1"} : std::vector<std::string>{"e0", "e1"},
-                                 "acc_v");
+                epilogue_emitter(em, r, names, "acc_v");
                 const std::string v = em.emit(r.epilogue)[0];
-                const std::string at = r.batched ? "(qbp * " + M + " + e0) * " + N + " + e1" : "e0 * " + N + " + e1";
                 e += body;
-                e += "        const int off = inb ? (int)((" + at + ") * 4) : (int)0x80000000;\n";
-                e += "        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, " + v +
-                     "), orsrc, off, 0, 0);\n    }\n";
+                const std::string i0 = buffered ? "e0" : "q0", i1 = buffered ? "e1" : "q1";
+                const std::string at = r.batched ? "(" + qbn + " * " + M + " + " + i0 + ") * " + N + " + " + i1
+                                                 : i0 + " * " + N + " + " + i1;
+                if (buffered) {
+                    e += "        const int off = inb ? (int)((" + at + ") * 4) : (int)0x80000000;\n";
+                    e += "        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, " + v +
+                         "), orsrc, off, 0, 0);\n";
+                    e += "    }\n";
+                }
+                else {
+                    e += "            out[" + at + "] = " + v + ";\n        }\n    }\n";
+                }
                 return e;
             };
-            s += "    const auto orsrc = __builtin_amdgcn_make_buffer_rsrc(out, 0, " +
-                 std::to_string(out_elems * 4) + ", 0x00020000);\n";
-            s += "    floatx16 accP[" + IB + "][2];\n";
-            s += "    #pragma unroll\n    for (int i = 0; i < " + IB + "; ++i)\n";
-            s += "        #pragma unroll\n        for (int j = 0; j < 2; ++j)\n";
-            s += "            #pragma unroll\n            for (int v = 0; v < 16; ++v) accP[i][j][v] = 0.0f;\n";
-            // the first tile has no predecessor: a row origin past the
-            // output masks every lane of its slices
-            s += "    idx_t m0p = " + std::to_string(r.m) + ";\n    idx_t n0p = 0;\n";
-            if (r.batched) s += "    idx_t qbp = 0;\n";
-            if (steps % 2 != 0) s += "    int phase = 0;\n";
-            s += "    for (idx_t rr = blockIdx.x; rr < " + std::to_string(total) + "; rr += gridDim.x) {\n";
-            s += decode("rr", "c", "    ");
-            s += "    const idx_t rn = rr + gridDim.x < " + std::to_string(total) + " ? rr + gridDim.x : rr;\n";
-            s += decode("rn", "x", "    ");
-            s += zero_acc;
-            // The next slice's global loads and LDS stores are issued in the
-            // same block as the MFMAs, so the scheduler can interleave both
-            // with them (the last step loads the workgroup's next tile).
+            if (persistent) {
+                s += "    const auto orsrc = __builtin_amdgcn_make_buffer_rsrc(out, 0, " +
+                     std::to_string(out_elems * 4) + ", 0x00020000);\n";
+                s += "    floatx16 accP[" + IB + "][2];\n";
+                s += "    #pragma unroll\n    for (int i = 0; i < " + IB + "; ++i)\n";
+                s += "        #pragma unroll\n        for (int j = 0; j < 2; ++j)\n";
+                s += "            #pragma unroll\n            for (int v = 0; v < 16; ++v) accP[i][j][v] = 0.0f;\n";
+                // the first tile has no predecessor: a row origin past the
+                // output masks every lane of its slices
+                s += "    idx_t m0p = " + std::to_string(r.m) + ";\n    idx_t n0p = 0;\n";
+                if (r.batched) s += "    idx_t qbp = 0;\n";
+                if (steps % 2 != 0) s += "    int phase = 0;\n";
+                s += "    for (idx_t rr = blockIdx.x; rr < " + std::to_string(total) + "; rr += gridDim.x) {\n";
+                s += decode("rr", "c", "    ");
+                s += "    const idx_t rn = rr + gridDim.x < " + std::to_string(total) + " ? rr + gridDim.x : rr;\n";
+                s += decode("rn", "x", "    ");
+            }
+            if (persistent) s += zero_acc;
+            // With both operands on the 128-bit path the next tile's global
+            // loads and LDS stores are issued in the same block as the
+            // MFMAs, so the scheduler can interleave both with them (the last
+            // step reloads its own tile, in bounds, into the idle buffer, or
+            // loads a persistent workgroup's next tile); otherwise they are
+            // skipped on the last step.
             std::string head;
-            head += steps % 2 != 0 ? "        const int cb = (phase + t) & 1;\n" : "        const int cb = t & 1;\n";
-            head += "        const int nb = cb ^ 1;\n";
-            head += "        const bool to_next = t + 1 == " + std::to_string(steps) + ";\n";
-            head += "        const idx_t k0 = to_next ? (idx_t)0 : (idx_t)(t + 1) * " + std::to_string(BK) + ";\n";
-            head += "        {\n";
-            head += "        const idx_t m0 = to_next ? m0x : m0c;\n";
-            head += "        const idx_t n0 = to_next ? n0x : n0c;\n";
-            head += "        const float* __restrict__ A = to_next ? Ax : Ac;\n";
-            head += "        const float* __restrict__ B = to_next ? Bx : Bc;\n";
-            head += load_a + load_b + "        }\n";
+            if (persistent) {
+                head += steps % 2 != 0 ? "        const int cb = (phase + t) & 1;\n" : "        const int cb = t & 1;\n";
+                head += "        const int nb = cb ^ 1;\n";
+                head += "        const bool to_next = t + 1 == " + std::to_string(steps) + ";\n";
+                head += "        const idx_t k0 = to_next ? (idx_t)0 : (idx_t)(t + 1) * " + std::to_string(BK) + ";\n";
+                head += "        {\n";
+                head += "        const idx_t m0 = to_next ? m0x : m0c;\n";
+                head += "        const idx_t n0 = to_next ? n0x : n0c;\n";
+                head += "        const float* __restrict__ A = to_next ? Ax : Ac;\n";
+                head += "        const float* __restrict__ B = to_next ? Bx : Bc;\n";
+                head += load_a + load_b + "        }\n";
+            }
+            else {
+                head += "        const int cb = t & 1;\n";
+                head += "        const int nb = cb ^ 1;\n";
+                if (interleave) {
+                    head += "        const idx_t k0 = (idx_t)(t + 1 < " + std::to_string(steps) +
+                            " ? t + 1 : t) * " + std::to_string(BK) + ";\n";
+                    head += "        {\n" + load_a + load_b + "        }\n";
+                }
+                else {
+                    head += "        const idx_t k0 = (idx_t)(t + 1) * " + std::to_string(BK) + ";\n";
+                    head += "        const bool more = t + 1 < " + std::to_string(steps) + ";\n";
+                    head += "        if (more) {\n" + load_a + load_b + "        }\n";
+                }
+            }
             std::string step;
             // this lane's k parity and row inside each 32-row block
             step += "        const int h = lane >> 5;\n";
@@ -458,81 +520,94 @@ namespace porch::cg {
             step += "                #pragma unroll\n                for (int j = 0; j < 2; ++j)\n";
             step += "                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i][st], bv[j][st], acc[i][j], 0, 0, 0);\n";
             // the LDS stores of the next slice, then the schedule; the
-            // two-ahead form picks its register set per step
+            // two-ahead persistent form picks its register set per step
             const std::string step_compute = step;
             step.clear();
             const int stores_per_step = static_cast<int>((2 * ib + steps - 1) / steps) * 16;
-            {
+            if (scheduled) {
                 // Instruction order for the scheduler: the 128-bit LDS reads
                 // first, then one of the next tile's global loads after every
                 // four MFMAs, so those loads leave early and their latency
-                // hides under the remaining MFMAs.  Then, after a gap of
-                // MFMAs that covers the loads' latency, one LDS store of the
-                // next tile after each MFMA, instead of all of them after the
-                // last MFMA.  The load groups name reads only (0x040): the
-                // previous tile's stores in the same block fill in around
-                // them.
+                // hides under the remaining MFMAs (measured 7% faster at
+                // 4096^3 than the compiler's own order, which issued them
+                // after nearly all MFMAs).  Then, after a gap of MFMAs that
+                // covers the loads' latency, one LDS store of the next tile
+                // after each MFMA, instead of all of them after the last
+                // MFMA (another 4% at 4096^3).  With the previous tile's
+                // stores in the same block the load groups name reads only
+                // (0x040); the stores fill in around them.
                 const int ds_reads = 2 * ib + 4;
+                const std::string vmem_mask = persistent ? "0x040" : "0x020";
                 step += "        __builtin_amdgcn_sched_group_barrier(0x100, " + std::to_string(ds_reads) + ", 0);\n";
                 for (int g = 0; g < vmem; ++g) {
                     step += "        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);\n";
-                    step += "        __builtin_amdgcn_sched_group_barrier(0x040, 1, 0);\n";
+                    step += "        __builtin_amdgcn_sched_group_barrier(" + vmem_mask + ", 1, 0);\n";
                 }
                 // the previous tile's output stores after this step's loads
                 if (ahead2)
                     step += "        __builtin_amdgcn_sched_group_barrier(0x080, " + std::to_string(stores_per_step) +
                             ", 0);\n";
                 int rest = mfmas - 4 * vmem;
-                const int gap = std::min(16, rest - ds_writes);
-                step += "        __builtin_amdgcn_sched_group_barrier(0x008, " + std::to_string(gap) + ", 0);\n";
-                for (int g = 0; g < ds_writes; ++g) {
-                    step += "        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);\n";
-                    step += "        __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);\n";
+                if (interleave) {
+                    const int gap = std::min(16, rest - ds_writes);
+                    step += "        __builtin_amdgcn_sched_group_barrier(0x008, " + std::to_string(gap) + ", 0);\n";
+                    for (int g = 0; g < ds_writes; ++g) {
+                        step += "        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);\n";
+                        step += "        __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);\n";
+                    }
+                    rest -= gap + ds_writes;
                 }
-                rest -= gap + ds_writes;
                 if (rest > 0)
                     step += "        __builtin_amdgcn_sched_group_barrier(0x008, " + std::to_string(rest) + ", 0);\n";
             }
+            if (!interleave) step += "        if (more) {\n" + store_a + store_b + "        }\n";
             step += "        __syncthreads();\n";
             const std::string step_schedule = step;
             auto step_of = [&](const std::string& lds_stores) {
-                return step_compute + "        {\n" + lds_stores + "        }\n" + step_schedule;
+                return step_compute + (interleave ? "        {\n" + lds_stores + "        }\n" : std::string()) +
+                       step_schedule;
             };
             step = step_of(store_a + store_b);
-            // steps unrolled, so each stores a fixed slice of the previous
-            // tile's accumulator blocks
-            for (int64_t t = 0; t < steps; ++t) {
-                const int lo = static_cast<int>(t * 2 * ib / steps);
-                const int hi = static_cast<int>((t + 1) * 2 * ib / steps);
-                s += "    {\n        const int t = " + std::to_string(t) + ";\n";
-                if (ahead2) {
-                    // load slice t + 2 (of this tile or the next) into set
-                    // t % 2; store slice t + 1 from the other set
-                    const bool next = t + 2 >= steps;
-                    const std::string sx = next ? "x" : "c";
-                    s += "        const int cb = t & 1;\n        const int nb = cb ^ 1;\n        {\n";
-                    s += "        const idx_t k0 = " + std::to_string(((t + 2) % steps) * BK) + ";\n";
-                    s += "        const idx_t m0 = m0" + sx + ";\n        const idx_t n0 = n0" + sx + ";\n";
-                    s += "        const float* __restrict__ A = A" + sx + ";\n";
-                    s += "        const float* __restrict__ B = B" + sx + ";\n";
-                    s += in_set(load_a + load_b, static_cast<int>(t % 2)) + "        }\n";
-                    s += epilogue(lo, hi);
-                    s += step_of(in_set(store_a + store_b, static_cast<int>((t + 1) % 2))) + "    }\n";
+            if (persistent) {
+                // steps unrolled, so each stores a fixed slice of the
+                // previous tile's accumulator blocks
+                for (int64_t t = 0; t < steps; ++t) {
+                    const int lo = static_cast<int>(t * 2 * ib / steps);
+                    const int hi = static_cast<int>((t + 1) * 2 * ib / steps);
+                    s += "    {\n        const int t = " + std::to_string(t) + ";\n";
+                    if (ahead2) {
+                        // load slice t + 2 (of this tile or the next) into
+                        // set t % 2; store slice t + 1 from the other set
+                        const bool next = t + 2 >= steps;
+                        const std::string sx = next ? "x" : "c";
+                        s += "        const int cb = t & 1;\n        const int nb = cb ^ 1;\n        {\n";
+                        s += "        const idx_t k0 = " + std::to_string(((t + 2) % steps) * BK) + ";\n";
+                        s += "        const idx_t m0 = m0" + sx + ";\n        const idx_t n0 = n0" + sx + ";\n";
+                        s += "        const float* __restrict__ A = A" + sx + ";\n";
+                        s += "        const float* __restrict__ B = B" + sx + ";\n";
+                        s += in_set(load_a + load_b, static_cast<int>(t % 2)) + "        }\n";
+                        s += epilogue("accP", "m0p", "n0p", "qbp", lo, hi, true);
+                        s += step_of(in_set(store_a + store_b, static_cast<int>((t + 1) % 2))) + "    }\n";
+                    }
+                    else {
+                        s += head;
+                        s += epilogue("accP", "m0p", "n0p", "qbp", lo, hi, true);
+                        s += step + "    }\n";
+                    }
                 }
-                else {
-                    s += head;
-                    s += epilogue(lo, hi);
-                    s += step + "    }\n";
-                }
+                if (steps % 2 != 0) s += "    phase += " + std::to_string(steps) + ";\n";
+                s += "    #pragma unroll\n    for (int i = 0; i < " + IB + "; ++i)\n";
+                s += "        #pragma unroll\n        for (int j = 0; j < 2; ++j) accP[i][j] = acc[i][j];\n";
+                s += "    m0p = m0c;\n    n0p = n0c;\n";
+                if (r.batched) s += "    qbp = qbc;\n";
+                s += "    }\n";
+                // the last tile's accumulators
+                s += epilogue("accP", "m0p", "n0p", "qbp", 0, 2 * ib, true);
             }
-            if (steps % 2 != 0) s += "    phase += " + std::to_string(steps) + ";\n";
-            s += "    #pragma unroll\n    for (int i = 0; i < " + IB + "; ++i)\n";
-            s += "        #pragma unroll\n        for (int j = 0; j < 2; ++j) accP[i][j] = acc[i][j];\n";
-            s += "    m0p = m0c;\n    n0p = n0c;\n";
-            if (r.batched) s += "    qbp = qbc;\n";
-            s += "    }\n";
-            // the last tile's accumulators
-            s += epilogue(0, 2 * ib);
+            else {
+                s += "    for (int t = 0; t < " + std::to_string(steps) + "; ++t) {\n" + head + step + "    }\n";
+                s += epilogue("acc", "m0", "n0", "qb", 0, 2 * ib, false);
+            }
             s += "}\n";
             return kc;
         }
@@ -547,11 +622,20 @@ namespace porch::cg {
         // with one short side that a skinny kernel serves better do not
         // get here).
         bool uses_mfma(const gemm_request& r) { return r.batch * r.m * r.n * r.k >= (int64_t{1} << 18); }
+
+        // Fewer than 16 values of K: fp32 MFMAs.  Split, each result is
+        // rounded six times where one to eight of them round it up to eight
+        // times: largest error over the sum of |a b|, fp32 / split, K = 1
+        // 6.0e-8 / 2.6e-7 (an outer product rounds correctly only here), K = 4
+        // 1.8e-7 / 2.5e-7, K = 12 2.3e-7 / 2.3e-7, K = 16 2.3e-7 / 1.7e-7.  And
+        // the stores bound them: 128 x 128 tiles over 1024 entries at K = 3 take
+        // 15.2 / 21.0 us, 3 x 10 matrices over 16384 entries 31 / 162.
+        bool uses_fp32(const gemm_request& r) { return r.k < 16 || fp32_persistent(r); }
     } // namespace
 
     kernel_code emit_gemm(const gemm_request& r) {
         if (!uses_mfma(r)) return emit_gemm_scalar(r);
-        return persistent(r) ? emit_gemm_persistent(r) : emit_gemm_split(r);
+        return uses_fp32(r) ? emit_gemm_fp32(r) : emit_gemm_split(r);
     }
 
     int64_t gemm_k_chunks(const gemm_request& r) {

@@ -193,3 +193,43 @@ def test_tiny_values_beside_ordinary_results(gpu):
     out = gpu.materialize(porch.matmul(gpu.tensor([m, k], a.reshape(-1)), gpu.tensor([k, n], b.reshape(-1))))
     exact = a.astype(np.float64) @ b.astype(np.float64)
     assert np.all(np.abs(out.cpu().reshape(m, n) - exact) <= k * 2.0 ** -24 * exact)
+
+
+# Below 16 values of K the fp32 MFMAs: no more than K roundings.  Aligned and
+# not, one tile a workgroup and persistent, 128- and 256-row tiles.
+SHORT = [(1, 700, 701, False), (2, 400, 390, True), (3, 300, 512, False), (4, 256, 300, False), (7, 200, 333, True),
+         (12, 180, 260, False), (15, 130, 141, True), (1, 4100, 4101, False), (4, 3900, 4000, False)]
+
+
+def short_k(make, k, m, n, transposed, rng):
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    b = rng.standard_normal((k, n)).astype(np.float32)
+    y = T(make(np.ascontiguousarray(b.T))) if transposed else make(b)
+    expr = porch.matmul(make(a), y)
+    (kernel,) = porch.plan(expr)["kernels"]
+    assert (kernel["kind"], kernel["block"]) == ("gemm.mfma", 256)
+    return a, b, expr
+
+
+def check_short(got, a, b):
+    exact = a.astype(np.float64) @ b.astype(np.float64)
+    scale = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    assert np.all(np.abs(got - exact) <= a.shape[1] * 2.0 ** -24 * scale)
+    if a.shape[1] == 1:
+        assert np.array_equal(got, a * b)
+
+
+@pytest.mark.skipif(not emu.available(), reason="no clang for the emulation")
+@pytest.mark.parametrize("case", [s for s in SHORT if s[0] in (1, 3, 15) and s[1] < 1000])
+def test_emulated_short_k(case):
+    a, b, expr = short_k(lambda x: filled(list(x.shape), x), *case, np.random.default_rng(9))
+    assert all(r["ok"] for r in emu.emulate(expr, timeout=300))
+    values = [a, np.ascontiguousarray(b.T) if case[3] else b]
+    check_short(emu.evaluate(expr, values, timeout=300).reshape(case[1], case[2]), a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", SHORT)
+def test_short_k(gpu, case):
+    a, b, expr = short_k(lambda x: gpu.tensor(list(x.shape), x.reshape(-1)), *case, np.random.default_rng(10))
+    check_short(gpu.materialize(expr).cpu().reshape(case[1], case[2]), a, b)
