@@ -630,7 +630,12 @@ namespace porch::cg {
         // 1.8e-7 / 2.5e-7, K = 12 2.3e-7 / 2.3e-7, K = 16 2.3e-7 / 1.7e-7.  And
         // the stores bound them: 128 x 128 tiles over 1024 entries at K = 3 take
         // 15.2 / 21.0 us, 3 x 10 matrices over 16384 entries 31 / 162.
-        bool uses_fp32(const gemm_request& r) { return r.k < 16 || fp32_persistent(r); }
+        // And products of 2^23 tiles and more: a launch holds fewer than 2^32
+        // threads, 256 a tile here and 512 for the split.
+        bool uses_fp32(const gemm_request& r) {
+            const int64_t tiles = ((r.m + BM - 1) / BM) * ((r.n + BN - 1) / BN) * r.batch;
+            return r.k < 16 || fp32_persistent(r) || tiles >= int64_t{1} << 23;
+        }
     } // namespace
 
     kernel_code emit_gemm(const gemm_request& r) {

@@ -233,3 +233,28 @@ def test_emulated_short_k(case):
 def test_short_k(gpu, case):
     a, b, expr = short_k(lambda x: gpu.tensor(list(x.shape), x.reshape(-1)), *case, np.random.default_rng(10))
     check_short(gpu.materialize(expr).cpu().reshape(case[1], case[2]), a, b)
+
+
+def test_plans_stay_within_a_launch():
+    # a launch holds fewer than 2^32 threads
+    for a, b in (([1 << 23, 17, 17], [1 << 23, 17, 17]), ([(1 << 23) + 5, 33, 49], [(1 << 23) + 5, 49, 33]),
+                 ([1 << 23, 9, 9], [1 << 23, 9, 9]), ([1 << 23, 10, 3], [1 << 23, 3, 10])):
+        expr = porch.batched_matmul(placeholder(a), placeholder(b))
+        (kernel,) = porch.plan(expr)["kernels"]
+        assert kernel["kind"] == "gemm.mfma" and kernel["grid"][0] * kernel["block"] < 1 << 32
+
+
+@pytest.mark.gpu
+def test_more_tiles_than_512_threads_each_can_be_launched_for(gpu):
+    # the same two 17 x 17 matrices for every entry, each product times a
+    # value of its own
+    rng = np.random.default_rng(14)
+    batch = (1 << 23) + 5
+    a, b = ints((1, 17, 17), rng), ints((1, 17, 17), rng)
+    x = rng.integers(1, 8, size=(batch, 1, 1)).astype(np.float32)
+    t = lambda v: gpu.tensor(list(v.shape), v.reshape(-1))
+    product = porch.batched_matmul(porch.broadcast_to(t(a), [batch, 17, 17]), porch.broadcast_to(t(b), [batch, 17, 17]))
+    expr = porch.sum(porch.sum(product * porch.broadcast_to(t(x), [batch, 17, 17]), 2), 1)
+    assert any(k["kind"] == "gemm.mfma" and k["grid"][0] == batch for k in gpu.plan(expr)["kernels"])
+    out = gpu.materialize(expr).cpu().reshape(batch)
+    assert np.array_equal(out, x.reshape(-1) * (a[0] @ b[0]).sum())
