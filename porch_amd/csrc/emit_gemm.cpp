@@ -630,11 +630,22 @@ namespace porch::cg {
         // 1.8e-7 / 2.5e-7, K = 12 2.3e-7 / 2.3e-7, K = 16 2.3e-7 / 1.7e-7.  And
         // the stores bound them: 128 x 128 tiles over 1024 entries at K = 3 take
         // 15.2 / 21.0 us, 3 x 10 matrices over 16384 entries 31 / 162.
+        // A tile or more for every compute unit, of K up to 48 or of small
+        // matrices (a side of 32 or less, the other and K at most 256): there
+        // the split's fixed cost a tile (2.2 us against 0.3, one workgroup a
+        // compute unit against two) outweighs its rate.  fp32 / split, 16384
+        // entries: 17 x 33 x 17 78 / 280 us, 17 x 128 x 40 343 / 475,
+        // 33 x 48 x 65 274 / 373, 100 x 17 x 41 196 / 304; 64 x 80 x 64 434 /
+        // 484, 33 x 100 x 65 615 / 481; 1024 of 17 x 512 x 40 111 / 89;
+        // 4096 x 48 x 4097 32.9 / 36.0.  With fewer tiles neither fills the
+        // chip and the split's shorter loop is even or ahead.
         // And products of 2^23 tiles and more: a launch holds fewer than 2^32
         // threads, 256 a tile here and 512 for the split.
         bool uses_fp32(const gemm_request& r) {
             const int64_t tiles = ((r.m + BM - 1) / BM) * ((r.n + BN - 1) / BN) * r.batch;
-            return r.k < 16 || fp32_persistent(r) || tiles >= int64_t{1} << 23;
+            const bool small = std::min(r.m, r.n) <= 32 && std::max({r.m, r.n, r.k}) <= 256;
+            return r.k < 16 || fp32_persistent(r) || tiles >= int64_t{1} << 23 ||
+                   (tiles >= std::max(r.compute_units, 1) && (r.k <= 48 || small));
         }
     } // namespace
 

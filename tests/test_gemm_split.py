@@ -258,3 +258,40 @@ def test_more_tiles_than_512_threads_each_can_be_launched_for(gpu):
     assert any(k["kind"] == "gemm.mfma" and k["grid"][0] == batch for k in gpu.plan(expr)["kernels"])
     out = gpu.materialize(expr).cpu().reshape(batch)
     assert np.array_equal(out, x.reshape(-1) * (a[0] @ b[0]).sum())
+
+
+# (batch, m, k, n, transposed B) on either side of the rule for many tiles: 256 tiles,
+# K of 48, small matrices of a side of 32 and K of 256; True: fp32 MFMAs
+MANY = [((256, 33, 48, 65, False), True), ((255, 33, 48, 65, False), False), ((256, 33, 49, 65, True), False),
+        ((256, 32, 80, 41, False), True), ((256, 33, 80, 41, False), False), ((256, 17, 255, 43, True), True),
+        ((256, 17, 257, 43, False), False), ((512, 9, 65, 201, False), True), ((1, 4097, 17, 4099, False), True)]
+
+
+def many(make, size, rng):
+    batch, m, k, n, transposed = size
+    a, b = ints((batch, m, k), rng), ints((batch, n, k) if transposed else (batch, k, n), rng)
+    y = porch.permute(make(b), [0, 2, 1]) if transposed else make(b)
+    return [a, b], porch.relu(porch.batched_matmul(make(a), y) - 3.0)
+
+
+@pytest.mark.parametrize("size, fp32", MANY)
+def test_many_tiles_plans(size, fp32):
+    _, expr = many(lambda x: placeholder(list(x.shape)), size, np.random.default_rng(11))
+    (kernel,) = porch.plan(expr)["kernels"]
+    assert (kernel["kind"], kernel["block"]) == ("gemm.mfma", 256 if fp32 else 512)
+
+
+@pytest.mark.skipif(not emu.available(), reason="no clang for the emulation")
+@pytest.mark.parametrize("size", [(256, 33, 48, 65, False), (256, 17, 255, 43, True)])
+def test_emulated_many_tiles(size):
+    values, expr = many(lambda x: filled(list(x.shape), x), size, np.random.default_rng(12))
+    want = host.evaluate(expr).reshape(size[0], size[1], size[3])
+    assert emu.check_edges(expr, values, want) == 4 * size[1] * size[3]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("size", [s for s, _ in MANY])
+def test_many_tiles(gpu, size):
+    _, expr = many(lambda x: gpu.tensor(list(x.shape), x.reshape(-1)), size, np.random.default_rng(13))
+    out = gpu.materialize(expr).cpu().reshape(expr.shape())
+    assert np.array_equal(out, host.evaluate(expr).reshape(out.shape))
