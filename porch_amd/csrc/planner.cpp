@@ -363,8 +363,9 @@ namespace porch::plan {
                 auto is = [&](int x, ir::op kind) { return x >= 0 && !temp_of.count(x) && g.at(x).kind == kind; };
                 // p = e / bcast(sum(e)), e = exp(f - bcast(max(f))): the
                 // softmax of ops.cpp, each node read only inside it
+                // (p times itself is p read as a matrix: it is made all the same)
                 const int p = g.at(pv).lhs;
-                if (!is(p, ir::op::divide) || !used_by(p, {pv})) return none;
+                if (!is(p, ir::op::divide) || !used_by(p, {pv}) || g.at(pv).rhs == p) return none;
                 const int e = g.at(p).lhs, sb = g.at(p).rhs;
                 if (!is(e, ir::op::exp) || !is(sb, ir::op::broadcast) || !used_by(sb, {p})) return none;
                 const int sum = g.at(sb).lhs, d = g.at(e).lhs;

@@ -143,6 +143,11 @@ def test_plans():
     assert "attention" not in kinds(both)
     both = porch.batched_matmul(p, v) + porch.broadcast_to(porch.max(s * 2.0, 2, True), [4, 128, d])
     assert "attention" not in kinds(both)
+    # the weights times themselves: they are made all the same, once
+    p = porch.softmax(porch.batched_matmul(P([4, 64, 64]), P([4, 64, 64])), 2)
+    assert "attention" not in kinds(porch.batched_matmul(p, p))
+    p = porch.softmax(porch.matmul(P([128, 128]), P([128, 128])), 1)
+    assert "attention" not in kinds(porch.matmul(p, p))
     # a softmax in all but its last step
     e = porch.exp(s - porch.broadcast_to(porch.max(s, 2, True), s.shape()))
     assert "attention" not in kinds(porch.batched_matmul(e, v))
