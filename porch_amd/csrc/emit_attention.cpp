@@ -330,6 +330,8 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
 
         // f of the 16 products sc[kb][..] of keys key0 + kb 32 + 8 g + 4 h + j
         const bool vec = vector_scores(*r.score_expr, r.score);
+        bool score_loads = false;
+        for (const int id : r.score_expr->postorder(r.score)) score_loads |= r.score_expr->at(id).op == kop::load;
         auto scores = [&](const std::string& sc, const std::string& key, bool masked, const std::string& ind) {
             std::string c = ind + "#pragma unroll\n" + ind + "for (int g = 0; g < 4; ++g) {\n";
             c += ind + "    const idx_t key = " + key + " + 8 * g + 4 * h;\n" + ind + "    (void)key;\n";
@@ -388,8 +390,8 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
         };
 
         // One wave a SIMD hides its own latencies: an MFMA, an LDS read,
-        // five vector instructions, and so on (8 heads of 2048 positions,
-        // dim 64: 102 us against 128 in the compiler's order).  With two
+        // six vector instructions, and so on (8 heads of 4096 positions,
+        // dim 64: 203 us, five instructions 262).  With two
         // waves a SIMD, or the longer products of dim 128, the compiler's
         // order is the faster one (16 heads of 4096: 365 us against 392).
         auto schedule = [&](const std::string& ind) {
@@ -399,7 +401,7 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
             for (int i = 0; i < 6 * DS * KB + 6 * (KT / 16) * DB; ++i) {
                 c += ind + "__builtin_amdgcn_sched_group_barrier(0x008, 1, 0);\n";
                 c += ind + "__builtin_amdgcn_sched_group_barrier(0x100, 1, 0);\n";
-                c += ind + "__builtin_amdgcn_sched_group_barrier(0x002, 5, 0);\n";
+                c += ind + "__builtin_amdgcn_sched_group_barrier(0x002, 6, 0);\n";
             }
             return c;
         };
@@ -425,9 +427,16 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
         // new maximum, the sum and the factor `alpha` for what came before
         auto weights = [&](const std::string& key0, bool masked, const std::string& pf, const std::string& ind) {
             std::string c;
+            // f's own loads behind the products: 48 heads of 1000 queries over
+            // 1023 keys with a mask 66 us against 90
+            if (split == 0 && D == 32 && waves == 8 && score_loads) c += ind + "__builtin_amdgcn_sched_barrier(0);\n";
             c += ind + "#pragma unroll\n" + ind + "for (int b = 0; b < " + KBS + "; ++b) {\n";
             c += scores("sc[b]", "(idx_t)(" + key0 + ") + b * 32", masked, ind + "    ");
             c += ind + "}\n";
+            // (see `own_tile`; shared tiles of dim 128 in eight waves, loads
+            // excepted: 32 heads of 1536 positions 225 us against 244)
+            if (split > 0 && D == 32) c += ind + "__builtin_amdgcn_sched_barrier(0);\n";
+            if (split == 0 && D == 128 && waves == 8) c += ind + "__builtin_amdgcn_sched_barrier(0x30);\n";
             c += ind + "float tm = sc[0][0];\n";
             c += ind + "#pragma unroll\n" + ind + "for (int b = 0; b < " + KBS + "; ++b)\n" + ind + "    #pragma unroll\n" + ind +
                  "    for (int v = 0; v < 16; ++v) tm = __builtin_fmaxf(tm, sc[b][v]);\n";
@@ -562,7 +571,13 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
                 c += ind + "    sc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[" + std::to_string(pr[0]) + "], qf[t][" +
                      std::to_string(pr[1]) + "], sc[b], 0, 0, 0);\n";
             c += ind + "}\n";
+            // V is split after the weights, and at dim 32 f's own loads come
+            // before them: in the compiler's order the weights wait for loads
+            // that they have no use for (64 heads of 32 queries over 4099 keys,
+            // dim 128 229 us against 149; 16 of 77 over 12288 with a mask, dim
+            // 32 162 against 131).
             c += weights("key0", masked, "pf", ind);
+            c += ind + "__builtin_amdgcn_sched_barrier(0);\n";
             c += ind + "#pragma unroll\n" + ind + "for (int d = 0; d < " + DBS + "; ++d) {\n";
             c += ind + "    porch_v16f own_sum;\n" + ind + "    #pragma unroll\n" + ind + "    for (int v = 0; v < 16; ++v) own_sum[v] = 0.0f;\n";
             c += ind + "    #pragma unroll\n" + ind + "    for (int t = 0; t < " + std::to_string(KT / 16) + "; ++t) {\n" + split8("vr[t][d]", "lowestV");
