@@ -220,8 +220,9 @@ porch_status porch_materialize(const porch_graph* graph,
  * it compiles and loads the graph's kernels (hipModuleLoadData allocates
  * code memory), may create the thread's stream, and on the first call on a
  * device looks up the array's address, which makes the runtime load the
- * array.  The same kernels run;
- * the graph's temporaries (memoised reductions, split-reduction partials,
+ * array.  The same kernels run, or where their temporaries need more than
+ * the array those of a plan with fewer (attention of few queries over many
+ * keys without its scores in memory); the graph's temporaries (memoised reductions, split-reduction partials,
  * materialised product operands) come from the fixed per-GPU array of
  * PORCH_NOALLOC_SCRATCH_BYTES, and a graph that needs more fails with
  * PORCH_ERR_INVALID_ARGUMENT.  Every call on a GPU shares that array:

@@ -331,8 +331,9 @@ namespace porch::capi {
         return guarded(body);
     }
 
-    prepared_graph prepare(const porch_graph* graph) {
-        const std::string key = table_key(graph);
+    prepared_graph prepare(const porch_graph* graph, bool lean) {
+        std::string key = table_key(graph);
+        if (lean && !key.empty()) key += "lean";
         prepared_graph entry;
         if (!key.empty()) {
             std::scoped_lock lock{tables().mutex};
@@ -354,7 +355,7 @@ namespace porch::capi {
         table.n_inputs = g.n_inputs;
         if (ir::checked_numel(root.out) > 0) {
             bool plan_hit = false;
-            table.plan = plan::lookup(ir::compact(g), &plan_hit);
+            table.plan = plan::lookup(ir::compact(g), &plan_hit, lean);
             entry.hit = plan_hit;
             if (!key.empty()) {
                 std::scoped_lock lock{tables().mutex};

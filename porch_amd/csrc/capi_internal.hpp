@@ -29,7 +29,8 @@ namespace porch::capi {
         int n_inputs = 0;
         bool hit = false; // served from a cache
     };
-    prepared_graph prepare(const porch_graph* graph);
+    // `lean`: planned without large temporaries where it can be (plan::build).
+    prepared_graph prepare(const porch_graph* graph, bool lean = false);
 
     // The runtime buffers behind the handles (null handles stay null).
     std::vector<rt::buffer_state*> input_states(const porch_buffer* const* inputs, int32_t n_inputs);

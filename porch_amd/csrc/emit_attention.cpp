@@ -204,20 +204,56 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
 )";
         }
 
+        // Two ways to share out the work.  Shared tiles: a workgroup walks all
+        // keys for 128 or 256 queries, its waves share each tile of K and V.
+        // Split keys: a workgroup takes a block of 32 queries, its waves share
+        // out the keys; each wave splits its own K and V into bf16 values, twice
+        // the vector work.  Times in us from the rounds of workgroups over the
+        // compute units and the tiles of 32 keys that a wave walks, per tile as
+        // measured (aligned, one stride over the batch; shared / split / the
+        // unfused program): dim 64, 1 x 1024 queries over 1024 keys 67 / 23 /
+        // 23, 16 x 2048 over 4096 275 / 290 / 570, 512 x 64 over 4096 662 / 355 /
+        // 937; dim 32, 4096 x 32 over 2048 1710 / 473 / 1539; dim 128, 40 x 300
+        // over 4096 363 / 273 / 332, 512 x 64 over 32 24.7 / 41 / 21.3.
+        struct shares {
+            int waves;
+            double us;
+        };
+
+        int64_t rounds_of(int64_t workgroups, int64_t resident) {
+            return (workgroups + resident - 1) / resident;
+        }
+
+        shares shared_tiles(int64_t batch, int64_t rows, int64_t keys, int64_t dim, int compute_units) {
+            const int64_t cus = std::max(compute_units, 8);
+            // Eight waves share each tile of K and V; four where that still
+            // leaves no compute unit a second workgroup.
+            const int waves = batch * ((rows + 127) / 128) <= cus ? 4 : 8;
+            const int64_t rounds = rounds_of(batch * ((rows + 32 * waves - 1) / (32 * waves)), cus);
+            const double tile = waves == 4 ? (dim == 32 ? 0.93 : dim == 64 ? 2.05 : 2.8) : (dim == 32 ? 1.65 : dim == 64 ? 2.35 : 6.0);
+            return {waves, 4.0 + static_cast<double>(rounds) * (1.5 + static_cast<double>((keys + 31) / 32) * tile)};
+        }
+
+        shares split_keys(int64_t batch, int64_t rows, int64_t keys, int64_t dim, int compute_units) {
+            const int64_t cus = std::max(compute_units, 8);
+            // (four waves fill a compute unit's registers at dim 128, half of
+            // them below)
+            const int waves = dim == 128 || keys <= 128 ? 4 : 8;
+            const int64_t rounds = rounds_of(batch * ((rows + 31) / 32), waves == 4 && dim < 128 ? 2 * cus : cus);
+            const int64_t tiles = ((keys + 31) / 32 + waves - 1) / waves;
+            const double tile = rounds == 1 ? (dim == 32 ? 2.2 : dim == 64 ? 3.7 : 4.0) : (dim == 32 ? 3.0 : dim == 64 ? 5.0 : 5.2);
+            const double fixed = dim == 128 ? 3.5 : (dim == 32 ? 0.5 : 1.5) + (waves == 8 ? dim == 32 ? 1.0 : 1.5 : 0.0);
+            return {waves, 4.0 + static_cast<double>(rounds) * (fixed + static_cast<double>(tiles) * tile)};
+        }
+
         // Waves among which the keys of a block of 32 queries are split; 0:
-        // none.  A workgroup of shared tiles walks all keys for 128 queries
-        // or more, which leaves compute units idle where there are few; with
-        // split keys each wave splits its own K and V into bf16 values, twice
-        // the vector work.  Shared / split, causal: dim 64, 8 heads of 128
-        // positions 14.8 / 9.9 us, 4 of 1000 (128 blocks) 89 / 32, 8 of 2048
-        // (512) 139 / 104; dim 32, 16 of 1000 (512) 76 / 32; dim 128, 4 of
-        // 2048 (256) 226 / 106, 24 of 512 (384) 70 / 71, 16 of 1000 (512) 116
-        // / 135: up to two rounds of blocks, one at dim 128, where four waves
-        // fill a compute unit's registers.
+        // none, shared tiles.
         int key_split(const attention_request& r) {
-            const int64_t blocks = r.batch * ((r.rows + 31) / 32);
-            if (blocks > (r.dim == 128 ? 1 : 2) * static_cast<int64_t>(std::max(r.compute_units, 8))) return 0;
-            return r.dim == 128 || r.keys <= 128 ? 4 : 8;
+            const shares split = split_keys(r.batch, r.rows, r.keys, r.dim, r.compute_units);
+            const double shared = shared_tiles(r.batch, r.rows, r.keys, r.dim, r.compute_units).us;
+            // (even: split up to two rounds of blocks, whose sums are the shorter ones)
+            const bool few = r.batch * ((r.rows + 31) / 32) <= 2 * static_cast<int64_t>(std::max(r.compute_units, 8));
+            return split.us < (few ? 1.08 : 1.0) * shared ? split.waves : 0;
         }
 
     } // namespace
@@ -228,6 +264,25 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
         return dim == value_dim && (dim == 32 || dim == 64 || dim == 128) && rows >= 32 && keys >= 32;
     }
 
+    bool attention_pays(int64_t batch, int64_t rows, int64_t keys, int64_t dim, int64_t copied, int compute_units) {
+        // No form splits the keys of a block of queries over workgroups, so
+        // that few queries over many keys run on a few compute units, where
+        // the products and the softmax of the unfused program use them all:
+        // dim 64, 1 x 32 queries over 16384 keys 241 us fused, 31 unfused; 8 x
+        // 256 over 16384 244 / 165; 64 x 32 over 4096 69 / 92.  The unfused
+        // program's launches and split products take 14 to 24 us, its
+        // scores (four passes over memory, and matrix cores that a tile of
+        // few rows leaves idle) 3.5 to 10.5 us a million, and each operand
+        // it can't read in place a copy.  It is taken where it is ahead by more
+        // than such an estimate is wrong by, and its scores take 1 GiB at most.
+        const double fused = std::min(shared_tiles(batch, rows, keys, dim, compute_units).us,
+                                      split_keys(batch, rows, keys, dim, compute_units).us);
+        const double score = rows < 100 ? (dim == 32 ? 4.3 : dim == 64 ? 8.5 : 10.5) : (dim == 32 ? 3.5 : dim == 64 ? 4.3 : 5.2);
+        const double unfused = (dim == 32 ? 16.0 : 19.0) + static_cast<double>(batch * rows) * static_cast<double>(keys) * score * 1e-6 +
+                               static_cast<double>(copied) * 8.0 / 4e6;
+        return fused <= 1.15 * unfused || batch * rows > (int64_t{1} << 28) / keys;
+    }
+
     kernel_code emit_attention(const attention_request& r) {
         if (!attention_fits(r.batch, r.rows, r.keys, r.dim, r.dim)) throw std::logic_error("emit_attention: shape");
         const int D = static_cast<int>(r.dim);
@@ -235,11 +290,8 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
         const int KT = key_split(r) > 0 ? 32 : std::max(32, 2048 / D);
         const int KB = KT / 32, DB = D / 32, DS = D / 16;
         const bool apart = D == 32; // see gather
-        // Eight waves (256 queries) a workgroup share each tile of K and V;
-        // four where that still leaves no compute unit a second workgroup.
-        const int64_t cus = std::max(r.compute_units, 8);
         const int split = key_split(r);
-        const int waves = split > 0 ? split : r.batch * ((r.rows + 127) / 128) <= cus ? 4 : 8;
+        const int waves = split > 0 ? split : shared_tiles(r.batch, r.rows, r.keys, r.dim, r.compute_units).waves;
         const int threads = 64 * waves;
         const int BQ = split > 0 ? 32 : 32 * waves;
         const int64_t tiles = (r.rows + BQ - 1) / BQ;

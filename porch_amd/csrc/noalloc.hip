@@ -2,7 +2,8 @@
 // output, allocating no device memory.  For callers that cannot call
 // hipMalloc (code under HIP graph capture, serving loops that forbid it).
 //
-// The kernels are the ones porch_materialize launches.  Their temporaries
+// The kernels are the ones porch_materialize launches, or where their
+// temporaries are too large those of a plan with fewer of them.  Temporaries
 // (memoised reductions, the partials of a split column reduction, product
 // operands materialised once) come from `scratch`, a fixed device array of
 // PORCH_NOALLOC_SCRATCH_BYTES that each GPU holds from the first call on it
@@ -65,13 +66,17 @@ extern "C" porch_status porch_materialize_noalloc(const porch_graph* graph,
                                                   int32_t* out_rank) {
     return porch::capi::guarded_call([&] {
         if (out == nullptr) throw std::invalid_argument("output buffer is null");
-        const porch::capi::prepared_graph entry = porch::capi::prepare(graph);
+        porch::capi::prepared_graph entry = porch::capi::prepare(graph);
         if (n_inputs < entry.n_inputs) throw std::invalid_argument("graph needs more input buffers");
         if (n_inputs > 0 && inputs == nullptr) throw std::invalid_argument("inputs are null");
         porch::capi::write_result_shape(entry.out_shape, out_shape, capacity, out_rank);
         if (entry.plan == nullptr) return; // empty result: nothing to write
         size_t need = 0;
         (void)porch::plan::workspace_layout(*entry.plan, &need);
+        if (need > PORCH_NOALLOC_SCRATCH_BYTES) {
+            entry = porch::capi::prepare(graph, true);
+            (void)porch::plan::workspace_layout(*entry.plan, &need);
+        }
         if (need > PORCH_NOALLOC_SCRATCH_BYTES)
             throw std::invalid_argument(
                 "porch_materialize_noalloc: the graph's temporaries need " + std::to_string(need) +

@@ -29,6 +29,7 @@ namespace porch::plan {
             const ir::graph& g;
             graph_plan& plan;
             int compute_units;
+            bool lean; // see build()
             std::map<int, int> temp_of;
             // Element offset of a node's values within its temporary (0
             // unless several nodes share one: the column softmax's max
@@ -39,8 +40,8 @@ namespace porch::plan {
             // The nodes that read each node.
             std::vector<std::vector<int>> users;
 
-            builder(const ir::graph& graph, graph_plan& target, int cus)
-                : g(graph), plan(target), compute_units(cus) {
+            builder(const ir::graph& graph, graph_plan& target, int cus, bool without_large_temporaries)
+                : g(graph), plan(target), compute_units(cus), lean(without_large_temporaries) {
                 users.resize(g.nodes.size());
                 for (size_t i = 0; i < g.nodes.size(); ++i) {
                     const ir::node& n = g.nodes[i];
@@ -402,8 +403,8 @@ namespace porch::plan {
             // An operand of shape [batch, rows, cols] read in place: one
             // stride over the batch, or one per level where the batch is two
             // axes merged (the heads of [batch, seq, heads, dim]: a copy of
-            // q, k and v each otherwise).
-            cg::gemm_operand attention_operand(int id, const std::vector<int64_t>& shape) {
+            // q, k and v each otherwise).  No slot: it can't be.
+            cg::gemm_operand in_place(int id, const std::vector<int64_t>& shape) {
                 if (shape.size() == 3 && pure_view_of_input(id)) {
                     auto affine = [&](int64_t inner) {
                         cg::kexpr k;
@@ -431,7 +432,11 @@ namespace porch::plan {
                         if (op.slot >= 0) return op;
                     }
                 }
-                return operand(id, shape);
+                return {};
+            }
+            cg::gemm_operand attention_operand(int id, const std::vector<int64_t>& shape) {
+                const cg::gemm_operand op = in_place(id, shape);
+                return op.slot >= 0 ? op : operand(id, shape);
             }
 
             bool try_attention(int id, arg_ref dest) {
@@ -446,7 +451,15 @@ namespace porch::plan {
                 const std::vector<int64_t>& qs = g.at(first.lhs).out;
                 const std::vector<int64_t>& ks = g.at(first.rhs).out;
                 const std::vector<int64_t>& vs = g.at(second.rhs).out;
-                if (!cg::attention_fits(batched ? qs[0] : 1, qs[o], ks[o + 1], qs[o + 1], vs[o + 1])) return false;
+                const int64_t batch = batched ? qs[0] : 1;
+                if (!cg::attention_fits(batch, qs[o], ks[o + 1], qs[o + 1], vs[o + 1])) return false;
+                int64_t copied = 0; // values the unfused products would copy first
+                for (const int x : {first.lhs, first.rhs, second.rhs}) {
+                    const std::vector<int64_t>& shape = g.at(x).out;
+                    const int64_t inner = in_place(x, shape).batch_inner;
+                    if (inner > 0 && inner < batch) copied += batch * shape[1] * shape[2];
+                }
+                if (!lean && !cg::attention_pays(batch, qs[o], ks[o + 1], qs[o + 1], copied, compute_units)) return false;
                 // other reductions and products that f or the epilogue read
                 std::set<int> others;
                 boundaries(found.f, others, {found.qk}, true);
@@ -458,7 +471,7 @@ namespace porch::plan {
                     if (depends_on(b, pv)) return false;
                 cg::attention_request r;
                 r.batched = batched;
-                r.batch = batched ? qs[0] : 1;
+                r.batch = batch;
                 r.rows = qs[o];
                 r.keys = ks[o + 1];
                 r.dim = qs[o + 1];
@@ -911,7 +924,7 @@ namespace porch::plan {
         return os.str();
     }
 
-    std::shared_ptr<graph_plan> build(const ir::graph& g, int compute_units) {
+    std::shared_ptr<graph_plan> build(const ir::graph& g, int compute_units, bool lean) {
         const auto start = std::chrono::steady_clock::now();
         auto plan = std::make_shared<graph_plan>();
         const ir::node& root = g.at(g.root());
@@ -924,7 +937,7 @@ namespace porch::plan {
                 need = std::max(need, ir::numel(n.shape));
             }
         }
-        builder b(g, *plan, compute_units);
+        builder b(g, *plan, compute_units, lean);
         if (ir::numel(root.out) > 0) b.emit(g.root(), {arg_ref::kind::output, 0});
         plan->codegen_ms = rt::elapsed_ms(start);
         return plan;
@@ -938,8 +951,8 @@ namespace porch::plan {
         plan.compile_ms = rt::elapsed_ms(start);
     }
 
-    std::shared_ptr<graph_plan> lookup(const ir::graph& g, bool* hit) {
-        const std::string key = ir::canonical_key(g);
+    std::shared_ptr<graph_plan> lookup(const ir::graph& g, bool* hit, bool lean) {
+        const std::string key = ir::canonical_key(g) + (lean ? "lean" : "");
         {
             std::scoped_lock lock{cache().mutex};
             auto found = cache().entries.find(key);
@@ -949,7 +962,7 @@ namespace porch::plan {
             }
         }
         if (hit) *hit = false;
-        std::shared_ptr<graph_plan> plan = build(g, planning_compute_units());
+        std::shared_ptr<graph_plan> plan = build(g, planning_compute_units(), lean);
         compile(*plan);
         {
             std::scoped_lock lock{rt::counters_mutex()};

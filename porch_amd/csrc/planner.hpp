@@ -62,13 +62,15 @@ namespace porch::plan {
         [[nodiscard]] std::string describe() const;
     };
 
-    // Plans (code generation only).
-    std::shared_ptr<graph_plan> build(const ir::graph& g, int compute_units);
+    // Plans (code generation only).  `lean`: of two programs for the same
+    // result the one without large temporaries, where that is the slower one
+    // (attention of few queries over many keys).
+    std::shared_ptr<graph_plan> build(const ir::graph& g, int compute_units, bool lean = false);
     // hiprtc for every step (no device needed).
     void compile(graph_plan& plan);
 
     // Cached plan for a compacted graph (plans and compiles on a miss).
-    std::shared_ptr<graph_plan> lookup(const ir::graph& g, bool* hit);
+    std::shared_ptr<graph_plan> lookup(const ir::graph& g, bool* hit, bool lean = false);
     void clear_cache();
 
     // Launches the plan on the calling thread's stream.  `inputs[i]` backs

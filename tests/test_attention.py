@@ -395,3 +395,27 @@ def test_faint_weights_of_large_values(gpu):
             q, k, v = faint_inputs(size, np.float32(value), 17)
             expr = graph(lambda x: gpu.tensor(list(x.shape), x.reshape(-1)), q, k, v, None)
             check_faint(gpu.materialize(expr).cpu().reshape(q.shape), q, k, v)
+
+
+# (batch, queries, keys, dim): few queries over many keys are left to the
+# products and the softmax, which use every compute unit
+@pytest.mark.parametrize("size, fused", [
+    ((1, 32, 262144, 64), False), ((8, 32, 32768, 64), False), ((8, 256, 16384, 64), False), ((4, 1000, 40000, 128), False),
+    ((1, 100, 4096, 32), False), ((64, 32, 4096, 64), True), ((16, 2048, 16384, 64), True), ((8, 256, 512, 64), True),
+    ((4096, 32, 4096, 32), True), ((1, 65536, 65536, 64), True)])
+def test_plans_of_few_queries(size, fused):
+    b, sq, sk, d = size
+    q, kv = placeholder([b, sq, d]), placeholder([b, sk, d])
+    assert (kinds(attention(q, kv, kv, 0.125)) == ["attention"]) == fused
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("size, fused", [((2, 33, 6000, 64, True), False), ((1, 100, 5001, 128, False), False),
+                                         ((3, 64, 4100, 32, True), False), ((1024, 32, 100, 64, False), True),
+                                         ((260, 64, 300, 128, True), True), ((520, 40, 70, 128, True), False)])
+def test_few_queries(gpu, size, fused):
+    q, k, v, mask = inputs(size, np.random.default_rng(18))
+    expr = graph(lambda x: gpu.tensor(list(x.shape), x.reshape(-1)), q, k, v, mask)
+    assert (kinds(expr) == ["attention"]) == fused
+    want, scale = reference(q, k, v, size[3] ** -0.5, mask)
+    close(gpu.materialize(expr).cpu().reshape(want.shape), want, scale)

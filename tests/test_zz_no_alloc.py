@@ -251,6 +251,23 @@ def test_rejects_temporaries_beyond_the_limit(gpu):
     assert np.isnan(values).all()  # nothing ran
 
 
+def test_a_plan_without_large_temporaries_takes_the_place_of_one_beyond_the_limit(gpu):
+    """Attention of few queries over many keys: its faster plan keeps the
+    scores, past the limit here; the other keeps none."""
+    q, kv = (porch.tensor(s, rand(s, 51 + i)) for i, s in enumerate(([1, 32, 64], [1, 1 << 18, 64])))
+    scores = porch.batched_matmul(q, porch.permute(kv, [0, 2, 1])) * 0.125
+    expr = porch.batched_matmul(porch.softmax(scores, 2), kv)
+    assert sum(max(t, 1) * 4 for t in porch.plan(expr)["temps"]) > LIMIT
+    want = porch.materialize(expr).cpu().reshape(expr.shape())
+    noalloc(expr)
+    calls = {}
+    got = noalloc(expr, calls)
+    assert not any(calls.values()), calls
+    # two orders of sums of 64 products inside exp, and of 2^18 weights of
+    # values of up to 5: within a few of the 2^-24 that each rounds by
+    assert np.all(np.abs(got - want) <= 64 * 2.0 ** -23 * 5)
+
+
 def test_rejects_a_short_output_buffer(gpu):
     expr = elementwise(4096, 41)
     status, message, values, _ = call_noalloc(expr, out_floats=4095)
