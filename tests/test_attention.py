@@ -419,3 +419,59 @@ def test_few_queries(gpu, size, fused):
     assert (kinds(expr) == ["attention"]) == fused
     want, scale = reference(q, k, v, size[3] ** -0.5, mask)
     close(gpu.materialize(expr).cpu().reshape(want.shape), want, scale)
+
+
+def part_inputs(batch, sq, dim, rng):
+    """One nonzero a query and a diagonal V over `dim` keys: a score is one
+    product, an output one weight times one value, all of 24 bits."""
+    value = lambda *shape: (rng.uniform(0.5, 1.0, shape) * rng.choice([-1.0, 1.0], shape)).astype(np.float32)
+    q = np.zeros((batch, sq, dim), np.float32)
+    q[:, np.arange(sq), np.arange(sq) % dim] = value(batch, sq)
+    k = value(batch, dim, dim)
+    v = np.zeros((batch, dim, dim), np.float32)
+    v[:, np.arange(dim), np.arange(dim)] = value(batch, dim)
+    return q, k, v
+
+
+def check_parts(got, q, k, v):
+    # Scores of at most 1, rounded once (2^-25); a weight's exponent (up to
+    # 2.9) rounded twice, exp2 within an ulp, a product and a quotient and the
+    # sum of up to 128 weights of one sign: below 16 roundings.  Without
+    # one of the six products of parts: 2^-18 or more.
+    want, _ = reference(q, k, v, 1.0)
+    nonzero = want != 0
+    assert np.all(got[~nonzero] == 0)
+    assert np.all(np.abs(got[nonzero] / want[nonzero] - 1) <= 16 * 2.0 ** -24)
+
+
+@pytest.mark.skipif(not emu.available(), reason="no clang for the emulation")
+@pytest.mark.parametrize("dim", [32, 64])
+def test_emulated_parts(dim):
+    q, k, v = part_inputs(1, 40, dim, np.random.default_rng(19))
+    expr = attention(host_only(q), host_only(k), host_only(v), 1.0)
+    assert kinds(expr) == ["attention"]
+    check_parts(emu.evaluate(expr, [q, k, v], timeout=300), q, k, v)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch, sq, dim", [(1, 40, 32), (1, 40, 64), (1, 40, 128), (19, 865, 32), (19, 865, 64),
+                                            (10, 831, 128), (40, 1000, 64)])
+def test_parts(gpu, batch, sq, dim):
+    q, k, v = part_inputs(batch, sq, dim, np.random.default_rng(20))
+    expr = attention(*(gpu.tensor(list(x.shape), x.reshape(-1)) for x in (q, k, v)), 1.0)
+    assert kinds(expr) == ["attention"]
+    check_parts(gpu.materialize(expr).cpu().reshape(q.shape), q, k, v)
+
+
+@pytest.mark.gpu
+def test_wide_indices(gpu):
+    # 2^30 scores: 64-bit indices, in shared tiles; the first, a middle and the
+    # last entry
+    size = (4, 16384, 16384, 32, False)
+    q, k, v, _ = inputs(size, np.random.default_rng(21))
+    expr = graph(lambda x: gpu.tensor(list(x.shape), x.reshape(-1)), q, k, v, None)
+    assert kinds(expr) == ["attention"] and "typedef long long idx_t" in gpu.kernel_source(expr, 0)
+    got = gpu.materialize(expr).cpu().reshape(q.shape)
+    for b, rows in ((0, slice(0, 200)), (2, slice(8000, 8200)), (3, slice(16184, 16384))):
+        want, scale = reference(q[b:b + 1, rows], k[b:b + 1], v[b:b + 1], size[3] ** -0.5)
+        close(got[b:b + 1, rows], want, scale)

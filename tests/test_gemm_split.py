@@ -295,3 +295,41 @@ def test_many_tiles(gpu, size):
     _, expr = many(lambda x: gpu.tensor(list(x.shape), x.reshape(-1)), size, np.random.default_rng(13))
     out = gpu.materialize(expr).cpu().reshape(expr.shape())
     assert np.array_equal(out, host.evaluate(expr).reshape(out.shape))
+
+
+# What each of the six products of parts adds, exactly: integers whose bits
+# reach into the second and third bf16 value of one side, or the second of
+# both, with sums below 2^24.  (name: bits of A, of B, nonzeros a column of B)
+PARTS = {"three values of A": (20, 1, 7), "three values of B": (1, 20, 7), "two values of either": (11, 11, 3)}
+
+
+def part_inputs(name, m, k, n, rng):
+    bits_a, bits_b, nonzeros = PARTS[name]
+    draw = lambda shape, bits: (rng.integers(1 << (bits - 1), 1 << bits, size=shape) * rng.choice([-1, 1], size=shape))
+    a = draw((m, k), bits_a).astype(np.float32)
+    b = np.zeros((k, n), np.float32)
+    for j in range(n):
+        b[rng.choice(k, nonzeros, replace=False), j] = draw(nonzeros, bits_b)
+    return a, b
+
+
+@pytest.mark.skipif(not emu.available(), reason="no clang for the emulation")
+@pytest.mark.parametrize("name", sorted(PARTS))
+def test_emulated_parts(name):
+    a, b = part_inputs(name, 100, 70, 90, np.random.default_rng(15))
+    expr = porch.matmul(filled([100, 70], a), filled([70, 90], b))
+    assert porch.plan(expr)["kernels"][0]["block"] == 512
+    got = emu.evaluate(expr, [a, b], timeout=300).reshape(100, 90)
+    assert np.array_equal(got, (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32))
+
+
+# one tile of 128 x 128, a K of one step and of 16, split K, 256 x 256 tiles
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", sorted(PARTS))
+def test_parts(gpu, name):
+    for m, k, n in [(100, 70, 90), (128, 16, 130), (500, 33, 200), (40, 1030, 37), (3901, 67, 3999)]:
+        a, b = part_inputs(name, m, k, n, np.random.default_rng(16))
+        expr = porch.matmul(gpu.tensor([m, k], a.reshape(-1)), gpu.tensor([k, n], b.reshape(-1)))
+        assert gpu.plan(expr)["kernels"][0]["block"] == 512
+        got = gpu.materialize(expr).cpu().reshape(m, n)
+        assert np.array_equal(got, (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32))
