@@ -638,13 +638,18 @@ namespace porch::cg {
         // 33 x 48 x 65 274 / 373, 100 x 17 x 41 196 / 304; 64 x 80 x 64 434 /
         // 484, 33 x 100 x 65 615 / 481; 1024 of 17 x 512 x 40 111 / 89;
         // 4096 x 48 x 4097 32.9 / 36.0.  With fewer tiles neither fills the
-        // chip and the split's shorter loop is even or ahead.
+        // chip and the split's shorter loop is even or ahead, but where both
+        // sides are 32 or less: this kernel skips the loads of the rows that a
+        // tile does not have, the split clamps them (A transposed, 16 entries:
+        // 16 x 176 x 27 7.0 / 10.8 us, 24 x 384 x 24 14.0 / 18.2; 33 x 176 x 33
+        // 16.7 / 11.1).
         // And products of 2^23 tiles and more: a launch holds fewer than 2^32
         // threads, 256 a tile here and 512 for the split.
         bool uses_fp32(const gemm_request& r) {
             const int64_t tiles = ((r.m + BM - 1) / BM) * ((r.n + BN - 1) / BN) * r.batch;
             const bool small = std::min(r.m, r.n) <= 32 && std::max({r.m, r.n, r.k}) <= 256;
-            return r.k < 16 || fp32_persistent(r) || tiles >= int64_t{1} << 23 ||
+            if (r.k_chunks > 1) return false;
+            return r.k < 16 || std::max(r.m, r.n) <= 32 || fp32_persistent(r) || tiles >= int64_t{1} << 23 ||
                    (tiles >= std::max(r.compute_units, 1) && (r.k <= 48 || small));
         }
     } // namespace

@@ -264,7 +264,8 @@ def test_more_tiles_than_512_threads_each_can_be_launched_for(gpu):
 # K of 48, small matrices of a side of 32 and K of 256; True: fp32 MFMAs
 MANY = [((256, 33, 48, 65, False), True), ((255, 33, 48, 65, False), False), ((256, 33, 49, 65, True), False),
         ((256, 32, 80, 41, False), True), ((256, 33, 80, 41, False), False), ((256, 17, 255, 43, True), True),
-        ((256, 17, 257, 43, False), False), ((512, 9, 65, 201, False), True), ((1, 4097, 17, 4099, False), True)]
+        ((256, 17, 257, 43, False), False), ((512, 9, 65, 201, False), True), ((1, 4097, 17, 4099, False), True),
+        ((16, 31, 389, 32, True), True), ((16, 33, 389, 32, True), False)]
 
 
 def many(make, size, rng):
