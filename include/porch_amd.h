@@ -222,7 +222,8 @@ porch_status porch_materialize(const porch_graph* graph,
  * device looks up the array's address, which makes the runtime load the
  * array.  The same kernels run, or where their temporaries need more than
  * the array those of a plan with fewer (attention of few queries over many
- * keys without its scores in memory); the graph's temporaries (memoised reductions, split-reduction partials,
+ * keys without its scores in memory, a long product in one piece); the
+ * graph's temporaries (memoised reductions, split-reduction partials,
  * materialised product operands) come from the fixed per-GPU array of
  * PORCH_NOALLOC_SCRATCH_BYTES, and a graph that needs more fails with
  * PORCH_ERR_INVALID_ARGUMENT.  Every call on a GPU shares that array:

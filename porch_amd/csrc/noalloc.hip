@@ -74,8 +74,13 @@ extern "C" porch_status porch_materialize_noalloc(const porch_graph* graph,
         size_t need = 0;
         (void)porch::plan::workspace_layout(*entry.plan, &need);
         if (need > PORCH_NOALLOC_SCRATCH_BYTES) {
-            entry = porch::capi::prepare(graph, true);
-            (void)porch::plan::workspace_layout(*entry.plan, &need);
+            const porch::capi::prepared_graph lean = porch::capi::prepare(graph, true);
+            size_t lean_need = 0;
+            (void)porch::plan::workspace_layout(*lean.plan, &lean_need);
+            if (lean_need <= PORCH_NOALLOC_SCRATCH_BYTES) {
+                entry = lean;
+                need = lean_need;
+            }
         }
         if (need > PORCH_NOALLOC_SCRATCH_BYTES)
             throw std::invalid_argument(

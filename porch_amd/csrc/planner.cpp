@@ -330,7 +330,7 @@ namespace porch::plan {
                     add_step(cg::emit_gemm_band(r), dest);
                     return true;
                 }
-                r.k_chunks = cg::gemm_k_chunks(r);
+                r.k_chunks = lean ? 1 : cg::gemm_k_chunks(r);
                 if (r.k_chunks > 1) {
                     // Too few tiles for the machine: chunks of K in
                     // parallel, their partial products summed after.

@@ -64,7 +64,7 @@ namespace porch::plan {
 
     // Plans (code generation only).  `lean`: of two programs for the same
     // result the one without large temporaries, where that is the slower one
-    // (attention of few queries over many keys).
+    // (attention of few queries over many keys, a product unsplit along K).
     std::shared_ptr<graph_plan> build(const ir::graph& g, int compute_units, bool lean = false);
     // hiprtc for every step (no device needed).
     void compile(graph_plan& plan);

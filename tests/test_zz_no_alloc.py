@@ -251,6 +251,13 @@ def test_rejects_temporaries_beyond_the_limit(gpu):
     assert np.isnan(values).all()  # nothing ran
 
 
+def test_a_product_in_one_piece_takes_the_place_of_partial_products_beyond_the_limit(gpu):
+    a, b = (np.random.default_rng(61).integers(-2, 3, s).astype(np.float32) for s in ((935, 36683), (36683, 1213)))
+    expr = porch.matmul(porch.tensor([935, 36683], a.reshape(-1)), porch.tensor([36683, 1213], b.reshape(-1)))
+    assert sum(max(t, 1) * 4 for t in porch.plan(expr)["temps"]) > LIMIT
+    assert_same(noalloc(expr), porch.materialize(expr).cpu())  # integers below 2^24: exact either way
+
+
 def test_a_plan_without_large_temporaries_takes_the_place_of_one_beyond_the_limit(gpu):
     """Attention of few queries over many keys: its faster plan keeps the
     scores, past the limit here; the other keeps none."""
