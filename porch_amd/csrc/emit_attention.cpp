@@ -252,7 +252,9 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
             const shares split = split_keys(r.batch, r.rows, r.keys, r.dim, r.compute_units);
             const double shared = shared_tiles(r.batch, r.rows, r.keys, r.dim, r.compute_units).us;
             // (even: split up to two rounds of blocks, whose sums are the shorter ones)
-            const bool few = r.batch * ((r.rows + 31) / 32) <= 2 * static_cast<int64_t>(std::max(r.compute_units, 8));
+            const int64_t blocks = r.batch * ((r.rows + 31) / 32);
+            const bool few = blocks <= 2 * static_cast<int64_t>(std::max(r.compute_units, 8));
+            if (blocks >= (int64_t{1} << 26) / split.waves) return 0; // 2^32 threads: past a launch
             return split.us < (few ? 1.08 : 1.0) * shared ? split.waves : 0;
         }
 

@@ -409,6 +409,14 @@ def test_plans_of_few_queries(size, fused):
     assert (kinds(attention(q, kv, kv, 0.125)) == ["attention"]) == fused
 
 
+@pytest.mark.parametrize("size", [(1 << 22, 64, 129, 32), (1 << 23, 64, 100, 64), ((1 << 23) - 1, 33, 32, 32)])
+def test_plans_of_many_queries_stay_within_a_launch(size):
+    b, sq, sk, d = size
+    q, kv = placeholder([b, sq, d]), placeholder([b, sk, d])
+    for kernel in porch.plan(attention(q, kv, kv, 0.125))["kernels"]:
+        assert kernel["grid"][0] * kernel["block"] < 1 << 32
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("size, fused", [((2, 33, 6000, 64, True), False), ((1, 100, 5001, 128, False), False),
                                          ((3, 64, 4100, 32, True), False), ((1024, 32, 100, 64, False), True),
