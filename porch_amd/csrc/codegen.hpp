@@ -26,9 +26,10 @@
 //   reduce.column_softmax  the same layout folding a softmax's max and sum
 //                    (relative to a moving anchor) in one read;
 //   gemm.mfma        products on the matrix cores: three bf16 values per fp32
-//                    one, or for many tiles of a short K persistent
-//                    workgroups on fp32 MFMAs, the elementwise epilogue
-//                    applied to the accumulators before the store;
+//                    one, or fp32 MFMAs for a short K and small matrices
+//                    (persistent workgroups over many aligned tiles), the
+//                    elementwise epilogue applied to the accumulators
+//                    before the store;
 //   attention        softmax of a product along its last axis, times a third
 //                    matrix, without the scores in memory;
 //   gemm.rows,       products with a few rows (or columns), streaming the

@@ -19,7 +19,9 @@
 // two halves of the wave.
 //
 // Few queries leave most of the chip idle that way: there the waves of a
-// workgroup split the keys of one block of 32 queries (see key_split).
+// workgroup split the keys of one block of 32 queries (see key_split), and
+// where even that leaves most of it idle the unfused program is the faster
+// one (see attention_pays).
 //
 // An iteration computes the products of the next tile, the weights of this
 // one and the sums of the one before: independent of each other, so that a
