@@ -250,9 +250,11 @@ namespace porch::cg {
     };
     // dim of 32, 64 or 128, 32 rows and keys or more, one launch's threads.
     bool attention_fits(int64_t batch, int64_t rows, int64_t keys, int64_t dim, int64_t value_dim);
-    // Whether one kernel is the faster program; `copied`: values of the
-    // operands that the unfused one would copy first.
-    bool attention_pays(int64_t batch, int64_t rows, int64_t keys, int64_t dim, int64_t copied, int compute_units);
+    // Whether one kernel is the faster program; `score_reads`: f reads more
+    // than the product (a mask); `copied`: values of the operands that the
+    // unfused program would copy first.
+    bool attention_pays(int64_t batch, int64_t rows, int64_t keys, int64_t dim, bool score_reads, int64_t copied,
+                        int compute_units);
     kernel_code emit_attention(const attention_request& request);
 
     // A short K (8 to 64, a multiple of 8) over 256 columns or more, A's

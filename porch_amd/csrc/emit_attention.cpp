@@ -249,15 +249,16 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
         }
 
         // Waves among which the keys of a block of 32 queries are split; 0:
-        // none, shared tiles.
-        int key_split(const attention_request& r) {
-            const shares split = split_keys(r.batch, r.rows, r.keys, r.dim, r.compute_units);
-            const double shared = shared_tiles(r.batch, r.rows, r.keys, r.dim, r.compute_units).us;
-            // (even: split up to two rounds of blocks, whose sums are the shorter ones)
-            const int64_t blocks = r.batch * ((r.rows + 31) / 32);
-            const bool few = blocks <= 2 * static_cast<int64_t>(std::max(r.compute_units, 8));
-            if (blocks >= (int64_t{1} << 26) / split.waves) return 0; // 2^32 threads: past a launch
-            return split.us < (few ? 1.08 : 1.0) * shared ? split.waves : 0;
+        // none, shared tiles.  Up to two rounds of blocks (one at dim 128) keys
+        // are split; past that only entries of few rows, which leave most of a
+        // workgroup's waves without queries, and where a launch holds the
+        // threads.
+        int key_split(int64_t batch, int64_t rows, int64_t keys, int64_t dim, int compute_units) {
+            const shares split = split_keys(batch, rows, keys, dim, compute_units);
+            const int64_t blocks = batch * ((rows + 31) / 32);
+            if (blocks >= (int64_t{1} << 26) / split.waves) return 0;
+            if (blocks <= (dim == 128 ? 1 : 2) * static_cast<int64_t>(std::max(compute_units, 8))) return split.waves;
+            return rows <= 128 && split.us < shared_tiles(batch, rows, keys, dim, compute_units).us ? split.waves : 0;
         }
 
     } // namespace
@@ -268,7 +269,8 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
         return dim == value_dim && (dim == 32 || dim == 64 || dim == 128) && rows >= 32 && keys >= 32;
     }
 
-    bool attention_pays(int64_t batch, int64_t rows, int64_t keys, int64_t dim, int64_t copied, int compute_units) {
+    bool attention_pays(int64_t batch, int64_t rows, int64_t keys, int64_t dim, bool score_reads, int64_t copied,
+                        int compute_units) {
         // No form splits the keys of a block of queries over workgroups, so
         // that few queries over many keys run on a few compute units, where
         // the products and the softmax of the unfused program use them all:
@@ -277,24 +279,38 @@ __device__ __forceinline__ int porch_row_dim(int p) { return (p & ~31) | ((p & 1
         // program's launches and split products take 14 to 24 us, its
         // scores (four passes over memory, and matrix cores that a tile of
         // few rows leaves idle) 3.5 to 10.5 us a million, and each operand
-        // it can't read in place a copy.  It is taken where it is ahead by more
-        // than such an estimate is wrong by, and its scores take 1 GiB at most.
-        const double fused = std::min(shared_tiles(batch, rows, keys, dim, compute_units).us,
-                                      split_keys(batch, rows, keys, dim, compute_units).us);
+        // it can't read in place a copy; a mask costs the kernel a fifth more (its
+        // rows are far apart) and the unfused program next to nothing.  That
+        // is taken where it is ahead by more than such an estimate is
+        // wrong by, up to 1 GiB of scores, for few queries from 1024 keys on
+        // (below, both take 20 to 30 us; at dim 128 past 512, from where on
+        // the second product is split along K) and for many entries of few rows;
+        // with about as many queries as keys and half the compute units at
+        // work the kernel's smaller error is worth more than the time (8
+        // heads of 1100, dim 128: 4.0e-7 against 4.8e-7, 94 us against 81).
+        const int64_t cus = std::max(compute_units, 8), blocks = batch * ((rows + 31) / 32);
+        const bool few = keys >= 1024 ? 2 * blocks < cus || keys >= 2 * rows : dim == 128 && keys > 512 && keys >= 2 * rows;
+        const bool short_rows = rows < 64 && blocks >= cus;
+        if (batch * rows > (int64_t{1} << 28) / keys || !(few || short_rows)) return true;
+        const shares form = key_split(batch, rows, keys, dim, compute_units) > 0
+                                ? split_keys(batch, rows, keys, dim, compute_units)
+                                : shared_tiles(batch, rows, keys, dim, compute_units);
+        const double fused = form.us * (score_reads ? 1.2 : 1.0);
+        const double launches = dim == 32 ? 14.5 : dim == 64 ? 18.0 : 20.0;
         const double score = rows < 100 ? (dim == 32 ? 4.3 : dim == 64 ? 8.5 : 10.5) : (dim == 32 ? 3.5 : dim == 64 ? 4.3 : 5.2);
-        const double unfused = (dim == 32 ? 16.0 : 19.0) + static_cast<double>(batch * rows) * static_cast<double>(keys) * score * 1e-6 +
+        const double unfused = launches + static_cast<double>(batch * rows) * static_cast<double>(keys) * score * 1e-6 +
                                static_cast<double>(copied) * 8.0 / 4e6;
-        return fused <= 1.15 * unfused || batch * rows > (int64_t{1} << 28) / keys;
+        return fused <= 1.08 * unfused;
     }
 
     kernel_code emit_attention(const attention_request& r) {
         if (!attention_fits(r.batch, r.rows, r.keys, r.dim, r.dim)) throw std::logic_error("emit_attention: shape");
         const int D = static_cast<int>(r.dim);
+        const int split = key_split(r.batch, r.rows, r.keys, r.dim, r.compute_units);
         // keys a tile: two buffers of K and V in 48 KB of LDS (96 at dim 128)
-        const int KT = key_split(r) > 0 ? 32 : std::max(32, 2048 / D);
+        const int KT = split > 0 ? 32 : std::max(32, 2048 / D);
         const int KB = KT / 32, DB = D / 32, DS = D / 16;
         const bool apart = D == 32; // see gather
-        const int split = key_split(r);
         const int waves = split > 0 ? split : shared_tiles(r.batch, r.rows, r.keys, r.dim, r.compute_units).waves;
         const int threads = 64 * waves;
         const int BQ = split > 0 ? 32 : 32 * waves;

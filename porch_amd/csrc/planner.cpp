@@ -459,7 +459,14 @@ namespace porch::plan {
                     const int64_t inner = in_place(x, shape).batch_inner;
                     if (inner > 0 && inner < batch) copied += batch * shape[1] * shape[2];
                 }
-                if (!lean && !cg::attention_pays(batch, qs[o], ks[o + 1], qs[o + 1], copied, compute_units)) return false;
+                std::set<int> seen;
+                std::function<bool(int)> reads = [&](int x) {
+                    if (x < 0 || x == found.qk || !seen.insert(x).second) return false;
+                    return temp_of.count(x) != 0 || is_boundary(g.at(x).kind) || g.at(x).kind == ir::op::input ||
+                           reads(g.at(x).lhs) || reads(g.at(x).rhs);
+                };
+                if (!lean && !cg::attention_pays(batch, qs[o], ks[o + 1], qs[o + 1], reads(found.f), copied, compute_units))
+                    return false;
                 // other reductions and products that f or the epilogue read
                 std::set<int> others;
                 boundaries(found.f, others, {found.qk}, true);

@@ -402,7 +402,8 @@ def test_faint_weights_of_large_values(gpu):
 @pytest.mark.parametrize("size, fused", [
     ((1, 32, 262144, 64), False), ((8, 32, 32768, 64), False), ((8, 256, 16384, 64), False), ((4, 1000, 40000, 128), False),
     ((1, 100, 4096, 32), False), ((64, 32, 4096, 64), True), ((16, 2048, 16384, 64), True), ((8, 256, 512, 64), True),
-    ((4096, 32, 4096, 32), True), ((1, 65536, 65536, 64), True)])
+    ((4096, 32, 4096, 32), True), ((1, 65536, 65536, 64), True), ((8, 32, 1000, 128), False), ((8, 32, 512, 128), True),
+    ((4, 1024, 1024, 128), True), ((4, 2048, 2048, 64), True), ((16, 520, 520, 32), True)])
 def test_plans_of_few_queries(size, fused):
     b, sq, sk, d = size
     q, kv = placeholder([b, sq, d]), placeholder([b, sk, d])
